@@ -789,9 +789,10 @@ static FieldDev upload_field(afe_ctx *ctx, const afe_field *f, DevBuf<double> &s
   FieldDev fd{0, 0, nullptr, nullptr, nullptr, 0.0};
   if (!f || f->n_modes <= 0) return fd;
   const int nm = f->n_modes, dim = f->dim;
+  // in half turns, as the kernels evaluate the modes
   std::vector<double> h((size_t)nm * dim + 2 * nm);
-  std::memcpy(h.data(), f->k, sizeof(double) * nm * dim);
-  std::memcpy(h.data() + nm * dim, f->phi, sizeof(double) * nm);
+  for (int i = 0; i < nm * dim; i++) h[i] = 2.0 * f->k[i];
+  for (int i = 0; i < nm; i++) h[nm * dim + i] = f->phi[i] / M_PI;
   std::memcpy(h.data() + nm * dim + nm, f->w, sizeof(double) * nm);
   store.upload(ctx, h);
   fd.n_modes = nm;
