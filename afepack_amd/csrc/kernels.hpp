@@ -465,64 +465,81 @@ __global__ __launch_bounds__(256) void k_gather_pair(int64_t n_rows, const int64
 // right-hand side: element load vectors, then a per-DOF gather in ascending
 // element order (Operator::L2Discretize, Operator.discretize.templates.h:80-152)
 // ---------------------------------------------------------------------------
-template <int KIND>
+// Basis values at a quadrature point from its reference barycentrics lam: the
+// elements are affine, so the physical point's barycentrics are the reference
+// ones and no element evaluates area ratios (a division each) at every point.
+template <int KIND> __device__ __forceinline__ void basis_at_bary(const double *lam, double *val) {
+  if constexpr (KIND == P2_TRI) {
+    val[0] = lam[0] * (2.0 * lam[0] - 1.0);
+    val[1] = lam[1] * (2.0 * lam[1] - 1.0);
+    val[2] = lam[2] * (2.0 * lam[2] - 1.0);
+    val[3] = 4.0 * lam[1] * lam[2];
+    val[4] = 4.0 * lam[0] * lam[2];
+    val[5] = 4.0 * lam[0] * lam[1];
+  } else {
+#pragma unroll
+    for (int j = 0; j < KindInfo<KIND>::NL; j++) val[j] = lam[j];
+  }
+}
+
+// FK is the right-hand side's kind: 0 and 1 the loads of the manufactured
+// solution prod_d sin(pi x_d) (constant and variable coefficient), 2 given at
+// the DOFs, 3 one.  One thread per element; FP64 VALU bound for 0 and 1, the
+// Fe store for 2 and 3.  2.1M P2 elements, 12 points, FK 0: 192 -> 66 us with
+// library sines and area ratios at every point before; 3.1M tetrahedra, 16
+// modes, FK 1: 1386 -> 311 us.
+template <int KIND, int FK>
 __global__ __launch_bounds__(256) void k_element_loads(
     int64_t n_elem, const double *__restrict__ coords, const int32_t *__restrict__ ev,
-    const int32_t *__restrict__ edof, const double *__restrict__ qd, int nq, int fkind,
+    const int32_t *__restrict__ edof, const double *__restrict__ qd, const double *__restrict__ qb, int nq,
     FieldDev fld, const double *__restrict__ nodal, double *__restrict__ Fe) {
   constexpr int D = KindInfo<KIND>::D, NL = KindInfo<KIND>::NL;
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n_elem) return;
   double v[D + 1][D];
   load_elem<KIND>(e, coords, ev, v);
-  const double volume = tmpl_volume<D>();
-  const double jac = l2g_jacobian<D>(v);
-  double F[NL];
+  const double jv = l2g_jacobian<D>(v) * tmpl_volume<D>();
+  double F[NL], nd[NL];
 #pragma unroll
-  for (int j = 0; j < NL; j++) F[j] = 0.0;
+  for (int j = 0; j < NL; j++) {
+    F[j] = 0.0;
+    if constexpr (FK == 2) nd[j] = nodal[edof[e * NL + j]];
+  }
   for (int l = 0; l < nq; l++) {
-    const double *q = qd + l * (D + 1);
-    double x[D];
-    local_to_global<D>(q, v, x);
-    double val[NL];
-    basis_val<KIND>(x, v, val);
-    double f;
-    if (fkind == 3) {
-      f = 1.0;
-    } else if (fkind == 2) {
+    const double *lam = qb + l * (D + 1);
+    double val[NL], f = 1.0;
+    basis_at_bary<KIND>(lam, val);
+    if constexpr (FK == 2) {
       f = 0.0;
 #pragma unroll
-      for (int j = 0; j < NL; j++) f += nodal[edof[e * NL + j]] * val[j];
-    } else {
-      double u = 1.0, gu[D], r[D], sn[D];
+      for (int j = 0; j < NL; j++) f = fma(nd[j], val[j], f);
+    } else if constexpr (FK < 2) {
+      double x[D], r[D], sn[D], u = 1.0;
+      bary_to_global<D>(lam, v, x);
 #pragma unroll
       for (int d = 0; d < D; d++) {
         r[d] = halfturn_reduce(x[d]);
         sn[d] = sinpi_reduced(r[d]);
         u *= sn[d];
       }
-      if (fkind == 0) {
-        f = D * M_PI * M_PI * u;
-      } else {
+      f = D * M_PI * M_PI * u;
+      if constexpr (FK == 1) {
+        double gg[D], dot = 0.0;
+        const double g = field_g<D, true>(fld, x, gg);
 #pragma unroll
         for (int d = 0; d < D; d++) {
           double gd = M_PI * cospi_reduced(r[d]);
 #pragma unroll
           for (int c = 0; c < D; c++)
             if (c != d) gd *= sn[c];
-          gu[d] = gd;
+          dot = fma(gg[d], gd, dot);
         }
-        double gg[D];
-        const double g = field_g<D, true>(fld, x, gg);
-        double dot = 0;
-#pragma unroll
-        for (int d = 0; d < D; d++) dot += gg[d] * gu[d];
-        f = exp(g) * (D * M_PI * M_PI * u - dot);
+        f = exp(g) * (f - dot);
       }
     }
-    const double Jxw = q[D] * jac * volume;
+    const double wf = qd[l * (D + 1) + D] * jv * f;
 #pragma unroll
-    for (int j = 0; j < NL; j++) F[j] += Jxw * f * val[j];
+    for (int j = 0; j < NL; j++) F[j] = fma(wf, val[j], F[j]);
   }
 #pragma unroll
   for (int j = 0; j < NL; j++) Fe[e * NL + j] = F[j];
@@ -630,15 +647,32 @@ __device__ __forceinline__ double element_error_qp(int64_t e, const double *__re
   return err;
 }
 
-__global__ __launch_bounds__(256) void k_gather_vec(int64_t n, int nl, const int64_t *__restrict__ adj_ptr,
+// f_i = sum of the row's element loads in ascending element order, one thread
+// per DOF.  The row's elements go in groups of VEC_GROUP, whose adjacency
+// entries, then loads, are fetched together (two dependent memory latencies a
+// group, not two an element).  With xcd = 1 each XCD takes a contiguous range
+// of DOFs, so that the loads of one element, 32 bytes on tetrahedra, reach one
+// L2 for the DOFs that share it.  0.53M DOFs of tetrahedra (24 elements each):
+// 336 -> 81 us; 4.2M P2 DOFs (3 each, round-robin blocks): 59 -> 46 us.
+constexpr int VEC_GROUP = 8;
+template <int NL>
+__global__ __launch_bounds__(256) void k_gather_vec(int64_t n, int xcd, const int64_t *__restrict__ adj_ptr,
                                                     const int32_t *__restrict__ adj,
                                                     const double *__restrict__ Fe, double *__restrict__ f) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = (int64_t)logical_block(xcd) * blockDim.x + threadIdx.x;
   if (i >= n) return;
   double s = 0.0;
-  for (int64_t p = adj_ptr[i]; p < adj_ptr[i + 1]; p++) {
-    const int32_t ea = adj[p];
-    s += Fe[(int64_t)(ea >> 3) * nl + (ea & 7)];
+  const int64_t p1 = adj_ptr[i + 1];
+  for (int64_t p = adj_ptr[i]; p < p1; p += VEC_GROUP) {
+    int32_t ea[VEC_GROUP];
+    double fe[VEC_GROUP];
+#pragma unroll
+    for (int g = 0; g < VEC_GROUP; g++) ea[g] = p + g < p1 ? adj[p + g] : -1;
+#pragma unroll
+    for (int g = 0; g < VEC_GROUP; g++) fe[g] = ea[g] >= 0 ? Fe[(int64_t)(ea[g] >> 3) * NL + (ea[g] & 7)] : 0.0;
+#pragma unroll
+    for (int g = 0; g < VEC_GROUP; g++)
+      if (ea[g] >= 0) s += fe[g];
   }
   f[i] = s;
 }
@@ -701,59 +735,6 @@ __global__ __launch_bounds__(256) void k_csr_diag(int64_t n, const int64_t *__re
   if (i < n) d[i] = val[rp[i]];
 }
 
-// ---------------------------------------------------------------------------
-// error functionals (Functional.templates.h:296-317,399-426): per-element
-// contributions, then a fixed-order reduction
-// ---------------------------------------------------------------------------
-template <int KIND>
-__global__ __launch_bounds__(256) void k_element_error(
-    int64_t n_elem, const double *__restrict__ coords, const int32_t *__restrict__ ev,
-    const int32_t *__restrict__ edof, const double *__restrict__ qd, int nq, int h1,
-    const double *__restrict__ uh, double *__restrict__ out) {
-  constexpr int D = KindInfo<KIND>::D, NL = KindInfo<KIND>::NL;
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n_elem) return;
-  double v[D + 1][D];
-  load_elem<KIND>(e, coords, ev, v);
-  const double volume = tmpl_volume<D>();
-  const double jac = l2g_jacobian<D>(v);
-  double u_loc[NL];
-#pragma unroll
-  for (int j = 0; j < NL; j++) u_loc[j] = uh[edof[e * NL + j]];
-  double err = 0.0;
-  for (int l = 0; l < nq; l++) {
-    const double *q = qd + l * (D + 1);
-    double x[D];
-    local_to_global<D>(q, v, x);
-    const double Jxw = q[D] * jac * volume;
-    if (!h1) {
-      double val[NL];
-      basis_val<KIND>(x, v, val);
-      double uhv = 0.0, ue = 1.0;
-#pragma unroll
-      for (int j = 0; j < NL; j++) uhv += u_loc[j] * val[j];
-#pragma unroll
-      for (int d = 0; d < D; d++) ue *= sin_pi(x[d]);
-      err += Jxw * (ue - uhv) * (ue - uhv);
-    } else {
-      double g[NL][D];
-      basis_grad<KIND>(x, v, g);
-#pragma unroll
-      for (int d = 0; d < D; d++) {
-        double gh = 0.0;
-#pragma unroll
-        for (int j = 0; j < NL; j++) gh += u_loc[j] * g[j][d];
-        double ge = M_PI * cos_pi(x[d]);
-#pragma unroll
-        for (int c = 0; c < D; c++)
-          if (c != d) ge *= sin_pi(x[c]);
-        err += Jxw * (gh - ge) * (gh - ge);
-      }
-    }
-  }
-  out[e] = err;
-}
-
 #pragma clang fp contract(on)
 
 // ---------------------------------------------------------------------------
@@ -769,18 +750,6 @@ __device__ inline double block_sum(double v, double *sh) {
   const double r = sh[0];
   __syncthreads();
   return r;
-}
-
-// partial sums of x over a fixed grid (grid-stride), one per block
-__global__ __launch_bounds__(256) void k_sum_partial(int64_t n, const double *__restrict__ x,
-                                                     double *__restrict__ part) {
-  __shared__ double sh[256];
-  double s = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    s += x[i];
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
 // out[k] = sum of part[k*stride + 0 .. np) for k < nsum, one block
@@ -833,6 +802,81 @@ __global__ __launch_bounds__(256) void k_error_qp_part(int64_t n_elem, const dou
     s += element_error_qp<KIND>(e, coords, ev, edof, qd, nq, h1, uh, exact);
   s = block_sum(s, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+
+// Functional::L2Error / H1SemiError against prod_d sin(pi x_d)
+// (Functional.templates.h:296-317,399-426): one grid-stride pass over the
+// elements, block sums in a fixed tree, gridDim.x partial sums.  The basis
+// comes from the points' reference barycentrics; the gradient of uh is
+// sum_i (d uh / d lam_i) grad lam_i, with the D + 1 gradients of the
+// barycentrics taken once per element.  FP64 VALU bound.  983K P2 elements,
+// 12 points: 49 us (H1) and 36 us (L2), each 123 us with an array of element
+// contributions, area ratios and library sines, and a second pass to add them.
+template <int KIND, int H1>
+__global__ __launch_bounds__(256) void k_error_part(int64_t n_elem, const double *__restrict__ coords,
+                                                    const int32_t *__restrict__ ev,
+                                                    const int32_t *__restrict__ edof,
+                                                    const double *__restrict__ qd, const double *__restrict__ qb,
+                                                    int nq, const double *__restrict__ uh,
+                                                    double *__restrict__ part) {
+  constexpr int D = KindInfo<KIND>::D, NL = KindInfo<KIND>::NL;
+  constexpr int P1KIND = D == 2 ? P1_TRI : P1_TET; // its basis is the barycentrics
+  __shared__ double sh[256];
+  double sum = 0.0;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n_elem;
+       e += (int64_t)gridDim.x * blockDim.x) {
+    double v[D + 1][D], u[NL], dl[D + 1][D], err = 0.0;
+    load_elem<KIND>(e, coords, ev, v);
+    const double jv = l2g_jacobian<D>(v) * tmpl_volume<D>();
+#pragma unroll
+    for (int j = 0; j < NL; j++) u[j] = uh[edof[e * NL + j]];
+    if constexpr (H1) basis_grad<P1KIND>(v[0], v, dl);
+    for (int l = 0; l < nq; l++) {
+      const double *lam = qb + l * (D + 1);
+      double x[D], sq = 0.0;
+      bary_to_global<D>(lam, v, x);
+      if constexpr (H1) {
+        double c[D + 1], r[D], sn[D];
+#pragma unroll
+        for (int i = 0; i <= D; i++) c[i] = u[i];
+        if constexpr (KIND == P2_TRI) {
+#pragma unroll
+          for (int i = 0; i < 3; i++) {
+            const int a = (i + 1) % 3, b = (i + 2) % 3;
+            // edge DOF 3 + k lies opposite vertex k: 4 lam_a lam_b
+            c[i] = fma(u[i], 4.0 * lam[i] - 1.0, 4.0 * fma(u[3 + a], lam[b], u[3 + b] * lam[a]));
+          }
+        }
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+          r[d] = halfturn_reduce(x[d]);
+          sn[d] = sinpi_reduced(r[d]);
+        }
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+          double ge = M_PI * cospi_reduced(r[d]), gh = 0.0;
+#pragma unroll
+          for (int k = 0; k < D; k++)
+            if (k != d) ge *= sn[k];
+#pragma unroll
+          for (int i = 0; i <= D; i++) gh = fma(c[i], dl[i][d], gh);
+          sq = fma(gh - ge, gh - ge, sq);
+        }
+      } else {
+        double val[NL], uhv = 0.0, ue = 1.0;
+        basis_at_bary<KIND>(lam, val);
+#pragma unroll
+        for (int j = 0; j < NL; j++) uhv = fma(u[j], val[j], uhv);
+#pragma unroll
+        for (int d = 0; d < D; d++) ue *= sin_pi(x[d]);
+        sq = (ue - uhv) * (ue - uhv);
+      }
+      err = fma(qd[l * (D + 1) + D], sq, err);
+    }
+    sum = fma(jv, err, sum);
+  }
+  sum = block_sum(sum, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = sum;
 }
 
 // out = sqrt(|sum of part[0 .. np)|), the sum in k_finalize's order and the

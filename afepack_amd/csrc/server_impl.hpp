@@ -577,6 +577,7 @@ extern "C" int afe_server_create(int32_t device, int64_t hbm_budget, int32_t max
   std::unique_ptr<afe_server> s(new afe_server);
   int rc = afe_ctx_create(device, &s->ctx);
   if (rc) return rc;
+  s->ctx->keep_scratch = false; // the budget counts the context's bytes
   if ((rc = afe_batch_create(s->ctx, AFE_PREC_FP32, smooth, &s->batch))) {
     afe_ctx_destroy(s->ctx);
     return rc;
