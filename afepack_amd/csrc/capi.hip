@@ -549,9 +549,12 @@ struct afe_space {
   std::vector<int64_t> gather_dep;
   bool distinct_dofs = false; // every element's DOFs are distinct (the batched gather)
   DevBuf<double> coords;
-  DevBuf<int32_t> ev, elem_dof, dof_mark, adj, col;
+  DevBuf<int32_t> ev, elem_dof, adj, col;
   DevBuf<int64_t> adj_ptr, rp;
   DevBuf<uint8_t> slot;
+  // zero Dirichlet elimination: the marked DOFs, and the positions of the
+  // off-diagonal entries in their rows and columns (k_boundary_positions)
+  DevBuf<int32_t> bnd_rows, bnd_pos;
 };
 
 // per 256-row block, the largest element adjacent to any row of blocks
@@ -612,12 +615,37 @@ extern "C" int afe_space_create_sides(afe_ctx *ctx, int32_t kind, int64_t n_vert
   s->coords.upload(ctx, s->h.coords);
   s->ev.upload(ctx, s->h.ev);
   s->elem_dof.upload(ctx, s->h.elem_dof);
-  s->dof_mark.upload(ctx, s->h.dof_mark);
   s->adj.upload(ctx, s->h.adj);
   s->adj_ptr.upload(ctx, s->h.adj_ptr);
   s->slot.upload(ctx, s->h.slot);
   s->rp.upload(ctx, s->h.rp);
   s->col.upload(ctx, s->h.col);
+  std::vector<int32_t> brows;
+  std::vector<int64_t> bptr;
+  std::vector<uint8_t> marked;
+  DevBuf<int64_t> d_bptr;
+  DevBuf<uint8_t> d_marked;
+  {
+    const Space &h = s->h;
+    int64_t np = 0;
+    marked.resize(h.n_dof);
+    for (int64_t i = 0; i < h.n_dof; i++) {
+      marked[i] = h.dof_mark[i] != 0;
+      if (!marked[i]) continue;
+      brows.push_back((int32_t)i);
+      bptr.push_back(np);
+      np += h.rp[i + 1] - h.rp[i] - 1;
+    }
+    if (!brows.empty()) {
+      s->bnd_rows.upload(ctx, brows);
+      s->bnd_pos.alloc(ctx, 2 * np);
+      d_bptr.upload(ctx, bptr);
+      d_marked.upload(ctx, marked);
+      k_boundary_positions<<<nblk((int64_t)brows.size() * BND_LANES), 256, 0, ctx->stream>>>(
+          (int64_t)brows.size(), s->bnd_rows.p, d_bptr.p, s->rp.p, s->col.p, d_marked.p, s->bnd_pos.p);
+      HIPCHK(hipGetLastError());
+    }
+  }
   HIPCHK(hipStreamSynchronize(ctx->stream));
   *out = s.release();
   API_END
@@ -1349,9 +1377,12 @@ extern "C" int afe_apply_dirichlet(afe_matrix *a, double *d_u, double *d_f) {
   std::lock_guard<CtxMutex> lk(a->ctx->mu);
   HIPCHK(hipSetDevice(a->ctx->device));
   afe_space *s = a->s;
-  k_dirichlet_zero<<<nblk(s->h.n_dof), 256, 0, a->ctx->stream>>>(s->h.n_dof, s->rp.p, s->col.p, s->dof_mark.p,
-                                                                  a->val.p, d_f);
-  HIPCHK(hipGetLastError());
+  const int64_t nr = (int64_t)s->bnd_rows.n, np = (int64_t)s->bnd_pos.n;
+  if (nr > 0) {
+    k_dirichlet_zero<<<nblk(std::max(nr, np)), 256, 0, a->ctx->stream>>>(nr, s->bnd_rows.p, s->rp.p, np, s->bnd_pos.p,
+                                                                        a->val.p, d_f);
+    HIPCHK(hipGetLastError());
+  }
   HIPCHK(hipStreamSynchronize(a->ctx->stream));
   API_END
 }
@@ -2321,12 +2352,13 @@ static int space_clone_into(afe_ctx *ctx, const afe_space *src, const double *co
   s->coords.upload(ctx, s->h.coords);
   clone_buf(ctx, s->ev, src->ev);
   clone_buf(ctx, s->elem_dof, src->elem_dof);
-  clone_buf(ctx, s->dof_mark, src->dof_mark);
   clone_buf(ctx, s->adj, src->adj);
   clone_buf(ctx, s->col, src->col);
   clone_buf(ctx, s->adj_ptr, src->adj_ptr);
   clone_buf(ctx, s->rp, src->rp);
   clone_buf(ctx, s->slot, src->slot);
+  clone_buf(ctx, s->bnd_rows, src->bnd_rows);
+  clone_buf(ctx, s->bnd_pos, src->bnd_pos);
   HIPCHK(hipStreamSynchronize(ctx->stream));
   *out = s.release();
   API_END
