@@ -387,6 +387,41 @@ Csr transpose(const Csr &a) {
   return t;
 }
 
+// Each thread takes a range of columns with about as many entries as the
+// others' and scans all of them, so every column is filled by one thread, row
+// after row.
+template <class K>
+void transpose_map(int64_t m, int64_t n, const std::vector<int64_t> &rp, const std::vector<int32_t> &col,
+                   std::vector<int64_t> &tptr, std::vector<int32_t> &trow, std::vector<K> &tk) {
+  const int64_t nnz = rp[m];
+  tptr.assign(n + 1, 0);
+  for (int64_t k = 0; k < nnz; k++) tptr[col[k] + 1]++;
+  for (int64_t j = 0; j < n; j++) tptr[j + 1] += tptr[j];
+  trow.resize(nnz);
+  tk.resize(nnz);
+#pragma omp parallel
+  {
+    const int64_t T = omp_get_num_threads(), t = omp_get_thread_num();
+    auto bound = [&](int64_t s) {
+      return s == T ? n : std::lower_bound(tptr.begin(), tptr.end(), nnz * s / T) - tptr.begin();
+    };
+    const int64_t j0 = bound(t), j1 = bound(t + 1);
+    std::vector<int64_t> fill(tptr.begin() + j0, tptr.begin() + std::max(j0, j1));
+    for (int64_t i = 0; i < m && j0 < j1; i++)
+      for (int64_t k = rp[i]; k < rp[i + 1]; k++) {
+        const int64_t j = col[k];
+        if (j < j0 || j >= j1) continue;
+        const int64_t p = fill[j - j0]++;
+        trow[p] = (int32_t)i;
+        tk[p] = (K)k;
+      }
+  }
+}
+template void transpose_map(int64_t, int64_t, const std::vector<int64_t> &, const std::vector<int32_t> &,
+                            std::vector<int64_t> &, std::vector<int32_t> &, std::vector<int32_t> &);
+template void transpose_map(int64_t, int64_t, const std::vector<int64_t> &, const std::vector<int32_t> &,
+                            std::vector<int64_t> &, std::vector<int32_t> &, std::vector<int64_t> &);
+
 // AMGSolver::getPMPt (src/AMGSolver.cpp:288-358): per coarse row, columns in
 // discovery order over P row x A row x P^T row with the diagonal first, then
 // compressed (diagonal first, rest ascending); each value accumulates

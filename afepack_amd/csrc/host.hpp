@@ -50,6 +50,12 @@ struct Csr {
   int64_t nnz() const { return rp.empty() ? 0 : rp[m]; }
 };
 
+// transposed index map of a CSR pattern: column j lists its entries' rows and
+// CSR positions from tptr[j] on, in ascending row order
+template <class K>
+void transpose_map(int64_t m, int64_t n, const std::vector<int64_t> &rp, const std::vector<int32_t> &col,
+                   std::vector<int64_t> &tptr, std::vector<int32_t> &trow, std::vector<K> &tk);
+
 struct Space {
   int kind = 0, tdim = 0, n_loc = 0, n_vtx = 0;
   int64_t n_vert = 0, n_elem = 0, n_dof = 0;
