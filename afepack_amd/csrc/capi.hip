@@ -2281,6 +2281,7 @@ extern "C" int afe_amg_destroy(afe_amg *g) {
 // the kept P (bit-identical to the host product), the layouts' values through
 // their source maps, and the coarsest inverse on the host from the new
 // coarsest values.  Layouts, launch tables and captured graphs stay valid.
+constexpr int64_t GAL_FEW_ROWS = 24576;
 static void device_lazy_refresh(afe_amg *g, afe_matrix *a) {
   afe_ctx *ctx = g->ctx;
   std::lock_guard<CtxMutex> lk(ctx->mu);
@@ -2295,8 +2296,15 @@ static void device_lazy_refresh(afe_amg *g, afe_matrix *a) {
     const int64_t *arp = l == 0 ? a->rp() : d.c_rp.p;
     const int32_t *acol = l == 0 ? a->col() : d.c_col.p;
     const int64_t nc = dn.n;
-    k_galerkin_rows<<<nblk(nc), 256, 0, s>>>(nc, d.P_rp.p, d.P_col.p, d.P_val.p, arp, acol, lvals(l), d.Pt_rp.p,
-                                              d.Pt_col.p, d.Pt_val.p, dn.c_rp.p, dn.c_col.p, dn.c_val.p);
+    auto go = [&](auto kern, int lanes) {
+      kern<<<nblk(nc * lanes), 256, 0, s>>>(nc, d.P_rp.p, d.P_col.p, d.P_val.p, arp, acol, lvals(l), d.Pt_rp.p,
+                                            d.Pt_col.p, d.Pt_val.p, dn.c_rp.p, dn.c_col.p, dn.c_val.p);
+    };
+    // 16 lanes for many rows of up to 48 entries on average (a lane owns up
+    // to four), 64 for longer rows and for levels of few rows, where a row's
+    // chain of loads is the time (3692 rows of 12 entries: 131 us with 16
+    // lanes, 52 with 64; 17115 rows 112 and 105; 68084 rows 87 us with 16)
+    nc > GAL_FEW_ROWS && h.A[l + 1].nnz() <= 48 * nc ? go(k_galerkin_rows<16>, 16) : go(k_galerkin_rows<64>, 64);
   }
   for (int l = 0; l < L; l++) {
     DevLevel &d = g->lv[l];
