@@ -408,7 +408,7 @@ template <class T> static void batch_issue_step(afe_batch *b, hipStream_t s) {
                                                     bp.tile);
   }
   const int lds_cap = (int)b->ctx->lds_bytes;
-  kb_tail<T><<<K, TAIL_THREADS, (size_t)lds_cap, s>>>(tj_buf<T>(b).p, tl_buf<T>(b).p, b->nu, lds_cap);
+  kb_tail<T><<<K, TAIL_THREADS, (size_t)lds_cap, s>>>(tj_buf<T>(b).p, tl_buf<T>(b).p, b->nu, 1, lds_cap);
   for (int l = L - 1; l >= 0; l--) {
     const BLaunch &bt = b->up_prolong[l];
     if (bt.grid) kb_prolong<T><<<bt.grid, BLK, 0, s>>>(S + bt.seg_off, bt.nseg, LV + bt.lv_off, LV + bt.lvn_off,

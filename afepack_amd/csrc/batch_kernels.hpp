@@ -151,9 +151,47 @@ template <class T> struct TailJob {
 template <class T>
 __global__ __launch_bounds__(TAIL_THREADS) void kb_tail(const TailJob<T> *__restrict__ jobs,
                                                         const LevelDev<T> *__restrict__ tl, int nu,
-                                                        int lds_cap) {
+                                                        int post_reverse, int lds_cap) {
   const TailJob<T> j = jobs[blockIdx.x];
-  tail_body<T>(tl + j.loff, j.l0, j.lc, j.minv, j.coarse_mode, nu, nu, 1, 7, lds_cap);
+  tail_body<T>(tl + j.loff, j.l0, j.lc, j.minv, j.coarse_mode, nu, nu, post_reverse, 7, lds_cap);
+}
+
+// ---- the cycle of the small levels as a matrix ------------------------------
+// Column c of the dense form of a sub-cycle is the sub-cycle applied to the
+// unit vector of row c.  Table and job of the columns [c0, c0 + m): every
+// column has its own vectors x | b | t per level in W (stride doubles a
+// column, cleared before), and its right-hand side is set here.
+__global__ __launch_bounds__(256) void k_dense_columns(int m, int c0, int nl, const LevelDev<double> *__restrict__ base,
+                                                       int64_t stride, double *__restrict__ W,
+                                                       LevelDev<double> *__restrict__ tl,
+                                                       TailJob<double> *__restrict__ jobs,
+                                                       const double *__restrict__ minv, int coarse_mode) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= m) return;
+  double *w = W + c * stride;
+  for (int l = 0; l < nl; l++) {
+    LevelDev<double> d = base[l];
+    d.x = w;
+    d.b = w + d.n;
+    d.t = w + 2 * (int64_t)d.n;
+    w += 3 * (int64_t)d.n;
+    if (l == 0) d.b[c0 + c] = 1.0;
+    tl[(int64_t)c * nl + l] = d;
+  }
+  jobs[c] = {minv, c * nl, 0, nl - 1, coarse_mode};
+}
+
+// B(i, c0 + c) = the column's x on the first level, through a 32 x 32 tile
+__global__ __launch_bounds__(256) void k_dense_store(int n, int m, int c0, int64_t stride,
+                                                     const double *__restrict__ W, double *__restrict__ B) {
+  __shared__ double tile[32][33];
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int i0 = blockIdx.x * 32, c1 = blockIdx.y * 32;
+  for (int k = ty; k < 32; k += 8)
+    if (c1 + k < m && i0 + tx < n) tile[k][tx] = W[(c1 + k) * stride + i0 + tx];
+  __syncthreads();
+  for (int k = ty; k < 32; k += 8)
+    if (i0 + k < n && c1 + tx < m) B[(int64_t)(i0 + k) * n + c0 + c1 + tx] = tile[tx][k];
 }
 
 // ---- CG kernels (natural numbering) ---------------------------------------

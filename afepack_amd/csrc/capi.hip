@@ -1694,6 +1694,15 @@ struct afe_amg {
   bool coarse_exact = true; // AMGSolver::isSolveMostProjectExactly()
   bool big_coarse = false; // dense coarsest level solved by k_coarse_gemv
   DevBuf<double> minv;
+  // the sub-cycle from dense_level down (from x = 0) as a matrix, for the
+  // stationary [0] and the symmetric [1] cycle; nu: the smoothing count it was
+  // built for, -1 when the values or the coarse solve changed since
+  int dense_level = -1;
+  bool dense_off = false; // its memory could not be allocated
+  struct Dense {
+    DevBuf<double> m;
+    int nu = -1;
+  } dense[2];
   DevBuf<LevelDev<double>> ld64;
   DevBuf<LevelDev<float>> ld32;
   std::vector<LevelDev<double>> h_ld64; // host copies of the level descriptors
@@ -1747,6 +1756,8 @@ static void drop_graphs(afe_amg *g) {
         e = nullptr;
       }
 }
+
+static void drop_dense(afe_amg *g) { g->dense[0].nu = g->dense[1].nu = -1; }
 
 // host CSR of the fine matrix (values from the device)
 static Csr fine_csr(afe_matrix *a) {
@@ -2004,6 +2015,89 @@ static void set_coarse_mode(afe_amg *g) {
   }
 }
 
+// The levels of at most DENSE_ROWS rows are applied as one matrix: a V-cycle
+// from x = 0 is linear in its right-hand side, and the sub-cycle from a small
+// level down is a chain of colour steps (115 a sweep on the levels of 2213 to
+// 33 rows of a 4225-DOF hierarchy) that no parallelism shortens, 50 to 500 us
+// in the single-workgroup tail, while the product with its matrix is one
+// launch: 2213^2 entries, 39 MB, 9 us.  Building it takes the tail's time once
+// per 256 columns (and again after new values), so the line lies where one
+// solve still gains: 21 stationary cycles on 4225 DOFs 11.4 ms without the
+// matrix, 4.9 / 3.1 / 1.7 ms with levels of up to 600 / 1100 / 2560 rows in it;
+// a moving-mesh step of 251K DOFs (refresh, matrix and 30 CG iterations) 9.30,
+// 8.71 / 8.05 / 8.03 ms, and 8.72 with 5000 rows.
+// AFE_DENSE_ROWS sets the bound for hierarchies built afterwards (0: none).
+constexpr int64_t DENSE_ROWS = 2560;
+static void choose_dense_level(afe_amg *g) {
+  const char *e = getenv("AFE_DENSE_ROWS");
+  const int64_t most = e ? std::strtoll(e, nullptr, 10) : DENSE_ROWS;
+  g->dense_level = -1;
+  drop_dense(g);
+  for (int l = 1; l < (int)g->lv.size(); l++)
+    if (g->lv[l].n <= most) {
+      g->dense_level = l;
+      break;
+    }
+}
+
+// whether cycles apply dense_level as a matrix.  When that is the coarsest
+// level its matrix is the dense inverse; a small one stays inside the tail
+// that runs the levels before it.  A cycle without smoothing has no colour
+// steps to save, and maps onto the coarsest space only, which the matrix's
+// rounding would leave.
+static bool dense_used(const afe_amg *g, int nu) {
+  const int ld = g->dense_level, Lc = (int)g->lv.size() - 1;
+  if (ld < 1 || nu == 0 || g->dense_off) return false;
+  if (ld < Lc) return true;
+  return g->coarse_mode == 0 && (g->tail0 == Lc || g->lv[Lc].n > COARSE_TAIL_MAX);
+}
+
+static const double *dense_matrix(const afe_amg *g, bool symmetric) {
+  return g->dense_level == (int)g->lv.size() - 1 ? g->minv.p : g->dense[symmetric ? 1 : 0].m.p;
+}
+
+// builds the matrix of the sub-cycle if it is used and not current: one
+// workgroup per column runs the tail's FP64 cycle on a unit vector
+static void ensure_dense(afe_amg *g, bool symmetric, int nu) {
+  const int ld = g->dense_level, L = (int)g->lv.size(), nl = L - ld;
+  if (!dense_used(g, nu) || ld == L - 1) return;
+  afe_amg::Dense &d = g->dense[symmetric ? 1 : 0];
+  if (d.nu == nu) return;
+  afe_ctx *ctx = g->ctx;
+  hipStream_t st = ctx->stream;
+  const int n = (int)g->lv[ld].n;
+  int64_t stride = 0;
+  for (int l = ld; l < L; l++) stride += 3 * g->lv[l].n;
+  // columns at a time: at most 256 MB of vectors
+  const int cols = (int)std::min<int64_t>(n, std::max<int64_t>(256, (int64_t(32) << 20) / stride));
+  DevBuf<LevelDev<double>> tl;
+  DevBuf<TailJob<double>> jobs;
+  DevBuf<double> own;
+  double *W;
+  try {
+    d.m.alloc(ctx, (size_t)n * n);
+    tl.alloc(ctx, (size_t)cols * nl);
+    jobs.alloc(ctx, cols);
+    W = call_scratch(ctx, (size_t)cols * stride, own);
+  } catch (const afe::Error &) { // no room: the levels stay as they are
+    g->dense_off = true;
+    drop_graphs(g);
+    return;
+  }
+  const int lds_cap = (int)ctx->lds_bytes;
+  for (int c0 = 0; c0 < n; c0 += cols) {
+    const int m = std::min(cols, n - c0);
+    k_fill<double><<<nblk(m * stride), 256, 0, st>>>(m * stride, W, 0.0);
+    k_dense_columns<<<nblk(m), 256, 0, st>>>(m, c0, nl, g->ld64.p + ld, stride, W, tl.p, jobs.p, g->minv.p,
+                                             g->coarse_mode);
+    kb_tail<double><<<m, TAIL_THREADS, (size_t)lds_cap, st>>>(jobs.p, tl.p, nu, symmetric ? 1 : 0, lds_cap);
+    k_dense_store<<<dim3(nblk(n, 32), nblk(m, 32)), 256, 0, st>>>(n, m, c0, stride, W, d.m.p);
+  }
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(st)); // before the tables go
+  d.nu = nu;
+}
+
 static void finish_levels(afe_amg *g);
 
 static void upload_layout(afe_amg *g, HostLayout &lay) {
@@ -2123,6 +2217,7 @@ static void upload_layout(afe_amg *g, HostLayout &lay) {
 static void finish_levels(afe_amg *g) {
   afe_ctx *ctx = g->ctx;
   const int L = (int)g->lv.size();
+  choose_dense_level(g);
   std::vector<LevelDev<double>> d64(L);
   std::vector<LevelDev<float>> d32(L);
   for (int l = 0; l < L; l++) {
@@ -2332,6 +2427,7 @@ static void device_lazy_refresh(afe_amg *g, afe_matrix *a) {
   HIPCHK(hipStreamSynchronize(s));
   g->A0 = a;
   g->host_vals_stale = true;
+  drop_dense(g);
 }
 
 // host copies of the level values after device refreshes
@@ -2631,13 +2727,15 @@ static void gs_colour(DevLevel &d, int c, hipStream_t st) {
 template <class T>
 static void issue_vcycle(afe_amg *g, int nu, bool symmetric, hipStream_t st, bool x0_zero) {
   const int Lc = (int)g->lv.size() - 1;
-  for (int l = 0; l < g->tail0; l++) {
+  const bool dense = dense_used(g, nu);
+  const int top = dense ? std::min(g->tail0, g->dense_level) : g->tail0; // levels run as launches
+  for (int l = 0; l < top; l++) {
     DevLevel &d = g->lv[l];
     DevLevel &dn = g->lv[l + 1];
     if (l == 0 && x0_zero && nu == 0) k_fill<T><<<nblk(d.n), 256, 0, st>>>(d.n, Prec<T>::x(d), (T)0);
     // the next level is smoothed by launches from zero: the restriction
     // takes its first colour step
-    const bool first_next = nu > 0 && l + 1 < g->tail0;
+    const bool first_next = nu > 0 && l + 1 < top;
     for (int it = 0; it < nu; it++)
       for (int c = 0; c < d.ncol; c++) {
         if (l == 0 && it == 0 && c == 0 && x0_zero) {
@@ -2671,20 +2769,22 @@ static void issue_vcycle(afe_amg *g, int nu, bool symmetric, hipStream_t st, boo
   }
   const int lds_cap = (int)g->ctx->lds_bytes; // dynamic LDS of the tail workgroup
   const size_t lds = (size_t)lds_cap;
-  if (g->big_coarse) {
-    DevLevel &dc = g->lv[Lc];
-    if (g->tail0 < Lc)
-      k_tail<T><<<1, TAIL_THREADS, lds, st>>>(Prec<T>::ld(g), g->tail0, Lc, g->minv.p, g->coarse_mode, nu, nu,
-                                               symmetric ? 1 : 0, 1, lds_cap);
-    k_coarse_gemv<T><<<nblk(dc.n, WPB), BLK, 0, st>>>((int)dc.n, g->minv.p, Prec<T>::b(dc), Prec<T>::x(dc));
-    if (g->tail0 < Lc)
-      k_tail<T><<<1, TAIL_THREADS, lds, st>>>(Prec<T>::ld(g), g->tail0, Lc, g->minv.p, g->coarse_mode, nu, nu,
-                                               symmetric ? 1 : 0, 4, lds_cap);
+  auto tail = [&](int lc, int phase) {
+    k_tail<T><<<1, TAIL_THREADS, lds, st>>>(Prec<T>::ld(g), g->tail0, lc, g->minv.p, g->coarse_mode, nu, nu,
+                                             symmetric ? 1 : 0, phase, lds_cap);
+  };
+  if (dense || g->big_coarse) {
+    // the levels of the tail above the dense one, its product, and back up
+    const int ld = dense ? g->dense_level : Lc;
+    DevLevel &dc = g->lv[ld];
+    if (g->tail0 < ld) tail(ld, 1);
+    k_coarse_gemv<T><<<nblk(dc.n, WPB), BLK, 0, st>>>((int)dc.n, dense ? dense_matrix(g, symmetric) : g->minv.p,
+                                                       Prec<T>::b(dc), Prec<T>::x(dc));
+    if (g->tail0 < ld) tail(ld, 4);
   } else {
-    k_tail<T><<<1, TAIL_THREADS, lds, st>>>(Prec<T>::ld(g), g->tail0, Lc, g->minv.p, g->coarse_mode, nu, nu,
-                                             symmetric ? 1 : 0, 7, lds_cap);
+    tail(Lc, 7);
   }
-  for (int l = g->tail0 - 1; l >= 0; l--) {
+  for (int l = top - 1; l >= 0; l--) {
     DevLevel &d = g->lv[l];
     DevLevel &dn = g->lv[l + 1];
     // the colour the post-smoother sweeps first is left to it
@@ -2732,6 +2832,7 @@ static bool use_graphs() {
 
 static void launch_graph_or_issue(afe_amg *g, int prec, bool symmetric, int nu) {
   hipStream_t st = g->ctx->stream;
+  ensure_dense(g, symmetric, nu);
   if (!use_graphs()) {
     if (prec == 1)
       issue_vcycle<float>(g, nu, symmetric, st, symmetric);
@@ -3213,6 +3314,7 @@ extern "C" int afe_amg_set_coarse_exact(afe_amg *g, int32_t exact) {
   std::lock_guard<CtxMutex> lk(g->ctx->mu);
   if ((exact != 0) != g->coarse_exact) {
     drop_graphs(g);
+    drop_dense(g);
     g->coarse_exact = exact != 0;
     set_coarse_mode(g);
   }

@@ -1,0 +1,80 @@
+"""GPU: the small levels' sub-cycle applied as a matrix against the same levels
+run step by step (AFE_DENSE_ROWS=0): the symmetric and the stationary cycle,
+one and three sweeps, coarsest level solved by the inverse or smoothed, a
+hierarchy whose every level below the first is in the matrix, one with tail
+levels above it and one with the tail off; then after new values, after another
+smoothing count and after the coarse solve changes.
+
+The matrix is the FP64 cycle's: FP64 results differ by rounding in sums of at
+most a few thousand terms (1e-12 relative bounds them, as in the other cycle
+tests); the FP32 cycle's levels round every step to 6e-8 relative, and its few
+hundred dependent steps differ by less than 1e-5.
+"""
+import numpy as np
+import pytest
+
+from tests.conftest import make_mesh
+
+pytestmark = pytest.mark.gpu
+
+
+def _pair(ctx, monkeypatch, A, prm, rows):
+    import afepack_amd as afe
+    monkeypatch.setenv("AFE_DENSE_ROWS", "0")
+    a = afe.Amg(A, prm)
+    monkeypatch.setenv("AFE_DENSE_ROWS", str(rows))
+    return a, afe.Amg(A, prm)
+
+
+def _compare(ctx, g0, g1, n, rng, f32=True):
+    import afepack_amd as afe
+    r = afe.DeviceVector.from_numpy(ctx, rng.uniform(-1, 1, n))
+    z = [afe.DeviceVector(ctx, n) for _ in range(2)]
+    for prec, tol in ((afe.PREC_FP64, 1e-12), (afe.PREC_FP32, 1e-5)):
+        for g, v in zip((g0, g1), z):
+            g.vcycle(v, r, prec)
+        a, b = (v.numpy() for v in z)
+        assert np.linalg.norm(a - b) <= tol * np.linalg.norm(a), prec
+    for g, v in zip((g0, g1), z):
+        v.zero()
+        g.precondition(v, r, 2)  # three stationary cycles
+    a, b = (v.numpy() for v in z)
+    assert np.linalg.norm(a - b) <= 1e-12 * np.linalg.norm(a)
+
+
+@pytest.mark.parametrize("kind,n,lazy,smooth,rows,tail", [
+    (1, 24, 0, 3, 2560, 4096), (1, 24, 0, 1, 100, 4096), (2, 20, 1, 1, 64, 0), (2, 20, 1, 2, 400, 4096),
+    (3, 9, 1, 1, 300, 4096), (3, 9, 1, 1, 2560, 0), (1, 60, 1, 1, 1100, 4096)])
+def test_matrix_form_equals_the_steps(ctx, monkeypatch, kind, n, lazy, smooth, rows, tail):
+    import afepack_amd as afe
+    print(f"case dense kind={kind} n={n} lazy={lazy} smooth={smooth} rows={rows} tail={tail}", flush=True)
+    c, ev, vm = make_mesh(kind, n, 0.05, 13)
+    sp = afe.Space(ctx, kind, c, ev, vm)
+    A = afe.Matrix(sp)
+    A.assemble(afe.OP_STIFF, 2)
+    b = sp.rhs(2, afe.F_POISSON)
+    A.apply_dirichlet(b)
+    g0, g1 = _pair(ctx, monkeypatch, A, afe.AmgParams(lazy=lazy, smooth=smooth, build_fp32=1), rows)
+    assert g1.info()["n"][-1] <= rows
+    for g in (g0, g1):
+        g.set_tail_rows(tail)
+    rng = np.random.default_rng(n)
+    _compare(ctx, g0, g1, sp.n_dof, rng)
+    xs = []
+    for g in (g0, g1):
+        x = afe.DeviceVector(ctx, sp.n_dof)
+        assert g.pcg(x, b, rtol=1e-10, max_it=300, prec=afe.PREC_FP32).converged == 1
+        xs.append(x.numpy())
+    assert np.linalg.norm(xs[0] - xs[1]) <= 1e-9 * np.linalg.norm(xs[0])
+    if lazy:  # new values on the pattern
+        A.assemble(afe.OP_VARSTIFF, 2, afe.field_random(4, 3 if kind == 3 else 2, 0.5, 3))
+        A.apply_dirichlet(b)
+        for g in (g0, g1):
+            g.lazy_reinit(A)
+        _compare(ctx, g0, g1, sp.n_dof, rng)
+    for g in (g0, g1):
+        g.set_smooth(2)
+    _compare(ctx, g0, g1, sp.n_dof, rng)
+    for g in (g0, g1):
+        g.set_coarse_exact(False)
+    _compare(ctx, g0, g1, sp.n_dof, rng)
