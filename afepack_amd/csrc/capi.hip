@@ -641,6 +641,9 @@ extern "C" int afe_space_create_sides(afe_ctx *ctx, int32_t kind, int64_t n_vert
       s->bnd_pos.alloc(ctx, 2 * np);
       d_bptr.upload(ctx, bptr);
       d_marked.upload(ctx, marked);
+      // a kernel right behind queued host copies stalls the call (3.8 ms at
+      // any size): the copies finish first
+      HIPCHK(hipStreamSynchronize(ctx->stream));
       k_boundary_positions<<<nblk((int64_t)brows.size() * BND_LANES), 256, 0, ctx->stream>>>(
           (int64_t)brows.size(), s->bnd_rows.p, d_bptr.p, s->rp.p, s->col.p, d_marked.p, s->bnd_pos.p);
       HIPCHK(hipGetLastError());
