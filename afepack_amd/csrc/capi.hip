@@ -342,6 +342,10 @@ extern "C" int afe_ctx_create(int device, afe_ctx **out) {
         (const void *)k_gather_staged<4, 2>, (const void *)k_gather_staged<4, 3>,
         (const void *)k_gather_staged<6, 0>, (const void *)k_gather_staged<6, 1>,
         (const void *)k_gather_staged<6, 2>, (const void *)k_gather_staged<6, 3>};
+    HIPCHK(hipFuncSetAttribute((const void *)k_sweep<float>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)c->lds_bytes));
+    HIPCHK(hipFuncSetAttribute((const void *)k_sweep<double>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)c->lds_bytes));
     for (const void *f : staged)
       HIPCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->lds_bytes));
   }
@@ -1655,6 +1659,21 @@ struct DevLevel {
   DevBuf<float> v32, invd32, diag32, p_v32, t_v32;
   DevBuf<double> x64, b64, t64;
   DevBuf<float> x32, b32, t32;
+  // whole sweeps as one launch (k_sweep): forward [0] and reverse [1]; nb = 0
+  // when the level runs one launch per colour.  y32 / y64: the second vector
+  // that the sweeps write while they read x, and the other way round
+  struct Sweep {
+    int nb = 0, ncol = 0, gs = 0;
+    int max_loc = 0, max_rows = 0, max_slices = 0, max_ent = 0;
+    DevBuf<SweepBlock> blocks;
+    DevBuf<int32_t> rows, col_slice, src;
+    DevBuf<SliceInfo> slices;
+    DevBuf<uint16_t> cols;
+    DevBuf<double> v64;
+    DevBuf<float> v32;
+  } sweep[2];
+  DevBuf<double> y64;
+  DevBuf<float> y32;
   std::vector<int32_t> perm; // new -> old
   bool stream = false;       // matrix larger than the caches: non-temporal loads
   // value-only refresh of a lazy hierarchy: the level's CSR (levels >= 1),
@@ -1798,6 +1817,7 @@ struct HostLevel {
   int cshift = 0;
   std::vector<int32_t> perm, iperm;
   std::vector<int32_t> smap, dsrc; // CSR entry -> layout position, row -> CSR diagonal
+  SweepTables sweep[2];            // blocks empty: one launch per colour
 };
 struct HostLayout {
   bool maps = false; // source maps for the value-only refresh
@@ -1857,14 +1877,44 @@ static void colour_code(HostLevel &hl) {
   hl.cshift = cshift;
 }
 
+// Levels whose sweeps run as one launch: of at most SWEEP_ROWS rows (larger
+// ones fill the chip with each colour and are bandwidth bound: with the bound at
+// 40K / 131K / 300K rows the CG of 263K P2 DOFs takes 9.02 / 9.03 / 9.66 ms,
+// the moving-mesh step of 251K P1 DOFs 6.78 / 6.65 / 6.86, the CG of 4.2M P2
+// DOFs 49.0 / 48.6 / 48.6 and 53.7 with its 481K-row level), of rows of at most SWEEP_ROW_ENTRIES entries on average and with
+// closures of at most SWEEP_FACTOR times the level (the Galerkin levels of
+// tetrahedra couple 40 rows and more: a block's closure there is a large part
+// of the level).  Levels inside the dense sub-cycle need none, nor do the
+// server's hierarchies, which its batch runs with shared launches.
+// AFE_SWEEP_ROWS sets the bound for hierarchies built afterwards (0: none).
+constexpr int64_t SWEEP_ROWS = 131072, SWEEP_ROW_ENTRIES = 24, SWEEP_BLOCK_MIN = 32, SWEEP_BLOCK_MAX = 320;
+constexpr double SWEEP_FACTOR = 6.0;
+static int64_t dense_rows_bound();
+
+static void build_sweeps(HostLevel &hl) {
+  const char *e = getenv("AFE_SWEEP_ROWS");
+  const int64_t most = e ? std::strtoll(e, nullptr, 10) : SWEEP_ROWS;
+  const int64_t n = hl.n;
+  if (t_first_fit_only || n > most || n <= dense_rows_bound() || hl.ncol < 2 || hl.ncol > 64 ||
+      (int64_t)hl.sa.cols.size() > SWEEP_ROW_ENTRIES * n)
+    return;
+  std::vector<int32_t> block_of;
+  // one block per CU
+  const int64_t target = std::min(SWEEP_BLOCK_MAX, std::max(SWEEP_BLOCK_MIN, (n + 255) / 256));
+  const int nb = sweep_partition(hl.sa, target, block_of);
+  if (!sweep_build(hl.sa, nb, block_of, false, SWEEP_FACTOR, hl.sweep[0]) ||
+      !sweep_build(hl.sa, nb, block_of, true, SWEEP_FACTOR, hl.sweep[1]))
+    hl.sweep[0] = hl.sweep[1] = SweepTables();
+}
+
 static void build_layout(const Hierarchy &h, HostLayout &lay, bool maps) {
   const int L = (int)h.A.size();
   lay.maps = maps && h.A[0].nnz() < INT32_MAX;
   lay.lv.assign(L, HostLevel());
   std::vector<std::vector<int32_t>> groups(L);
   // phase times for AFE_VERBOSE: colouring, row order, level sliced ELL,
-  // transfer operators, natural copy
-  double tph[5] = {0, 0, 0, 0, 0};
+  // transfer operators, natural copy, sweep blocks
+  double tph[6] = {0, 0, 0, 0, 0, 0};
   auto tick = [t = std::chrono::steady_clock::now()](double &acc) mutable {
     const auto now = std::chrono::steady_clock::now();
     acc += std::chrono::duration<double>(now - t).count();
@@ -1928,6 +1978,8 @@ static void build_layout(const Hierarchy &h, HostLayout &lay, bool maps) {
     if ((int64_t)hl.sa.cols.size() * 8 > stream_bytes() && hl.ncol <= CC_BASES && getenv("AFE_NO_C16") == nullptr)
       colour_code(hl);
     tick(tph[2]);
+    if (l + 1 < L) build_sweeps(hl);
+    tick(tph[5]);
     if (l + 1 < L) {
       build_sell(h.P[l], lay.lv[l + 1].perm, hl.iperm, {(int32_t)h.P[l].m}, false, hl.sp, nullptr, nullptr,
                  l == 0 ? 0 : lane_shift(h.P[l].m, 1, h.P[l].nnz()));
@@ -1990,8 +2042,10 @@ static void build_layout(const Hierarchy &h, HostLayout &lay, bool maps) {
     tick(tph[4]);
   }
   if (verbose())
-    fprintf(stderr, "layout: colouring %.3f s, row order %.3f s, level ELL %.3f s, transfer %.3f s, natural %.3f s\n",
-            tph[0], tph[1], tph[2], tph[3], tph[4]);
+    fprintf(stderr,
+            "layout: colouring %.3f s, row order %.3f s, level ELL %.3f s, transfer %.3f s, natural %.3f s, "
+            "sweep blocks %.3f s\n",
+            tph[0], tph[1], tph[2], tph[3], tph[4], tph[5]);
   if (h.full) {
     // the coarse vectors are in the level's colour order: permute the inverse
     const std::vector<int32_t> &pc = lay.lv[L - 1].perm;
@@ -2031,9 +2085,13 @@ static void set_coarse_mode(afe_amg *g) {
 // 8.71 / 8.05 / 8.03 ms, and 8.72 with 5000 rows.
 // AFE_DENSE_ROWS sets the bound for hierarchies built afterwards (0: none).
 constexpr int64_t DENSE_ROWS = 2560;
-static void choose_dense_level(afe_amg *g) {
+static int64_t dense_rows_bound() {
   const char *e = getenv("AFE_DENSE_ROWS");
-  const int64_t most = e ? std::strtoll(e, nullptr, 10) : DENSE_ROWS;
+  return e ? std::strtoll(e, nullptr, 10) : DENSE_ROWS;
+}
+
+static void choose_dense_level(afe_amg *g) {
+  const int64_t most = dense_rows_bound();
   g->dense_level = -1;
   drop_dense(g);
   for (int l = 1; l < (int)g->lv.size(); l++)
@@ -2101,6 +2159,39 @@ static void ensure_dense(afe_amg *g, bool symmetric, int nu) {
   d.nu = nu;
 }
 
+// the blocks' value arrays and the second level vector
+static void alloc_sweeps(afe_amg *g, DevLevel &d) {
+  for (DevLevel::Sweep &w : d.sweep) {
+    if (w.nb == 0) continue;
+    w.v64.alloc(g->ctx, w.src.n);
+    d.y64.alloc(g->ctx, d.n);
+    if (g->has32) {
+      w.v32.alloc(g->ctx, w.src.n);
+      d.y32.alloc(g->ctx, d.n);
+    }
+  }
+}
+
+// the blocks' values from the level's current ones
+static void fill_sweeps(afe_amg *g, DevLevel &d) {
+  for (DevLevel::Sweep &w : d.sweep)
+    if (w.nb > 0)
+      k_sweep_values<<<nblk(w.src.n), 256, 0, g->ctx->stream>>>((int64_t)w.src.n, w.src.p, d.v64.p, w.v64.p, d.v32.p,
+                                                                w.v32.p);
+  HIPCHK(hipGetLastError());
+}
+
+template <class T> static SweepLds sweep_lds_of(const DevLevel::Sweep &w) {
+  return sweep_lds<T>(w.max_loc, w.max_rows, w.max_slices, w.ncol, w.max_ent);
+}
+
+// whether level d's sweeps run as one launch in precision T
+template <class T> static bool sweeps_fused(const afe_amg *g, const DevLevel &d) {
+  for (const DevLevel::Sweep &w : d.sweep)
+    if (w.nb == 0 || sweep_lds_of<T>(w).total > g->ctx->lds_bytes) return false;
+  return true;
+}
+
 static void finish_levels(afe_amg *g);
 
 static void upload_layout(afe_amg *g, HostLayout &lay) {
@@ -2154,6 +2245,25 @@ static void upload_layout(afe_amg *g, HostLayout &lay) {
         d.t_v32.upload(ctx, to_prec<float>(st.vals));
       }
     }
+    for (int k = 0; k < 2; k++) {
+      const SweepTables &t = hl.sweep[k];
+      DevLevel::Sweep &w = d.sweep[k];
+      w.nb = (int)t.blocks.size();
+      if (w.nb == 0) continue;
+      w.ncol = t.ncol;
+      w.gs = t.gshift;
+      w.max_loc = t.max_loc;
+      w.max_rows = t.max_rows;
+      w.max_slices = t.max_slices;
+      w.max_ent = t.max_ent;
+      w.blocks.upload(ctx, t.blocks);
+      w.rows.upload(ctx, t.rows);
+      w.slices.upload(ctx, t.slices);
+      w.col_slice.upload(ctx, t.col_slice);
+      w.cols.upload(ctx, t.cols);
+      w.src.upload(ctx, t.src);
+    }
+    alloc_sweeps(g, d);
     d.x64.alloc(ctx, d.n);
     d.b64.alloc(ctx, d.n);
     d.t64.alloc(ctx, d.n);
@@ -2212,7 +2322,9 @@ static void upload_layout(afe_amg *g, HostLayout &lay) {
   g->tail0 = L - 1;
   while (g->tail0 > 0 && g->lv[g->tail0 - 1].n <= g_tune.tail_rows) g->tail0--;
   if (h.full) g->minv.upload(ctx, lay.minv_perm);
-  finish_levels(g);
+  finish_levels(g); // returns with the copies finished
+  for (DevLevel &d : g->lv) fill_sweeps(g, d);
+  HIPCHK(hipStreamSynchronize(ctx->stream));
 }
 
 // the level descriptors of the tail and batch kernels (device pointers into
@@ -2410,6 +2522,7 @@ static void device_lazy_refresh(afe_amg *g, afe_matrix *a) {
     k_refresh_vals<<<nblk(nnz), 256, 0, s>>>(nnz, lvals(l), d.smap.p, d.v64.p, g->has32 ? d.v32.p : nullptr);
     k_refresh_diag<<<nblk(d.n), 256, 0, s>>>(d.n, lvals(l), d.dsrc.p, d.diag64.p, d.invd64.p,
                                              g->has32 ? d.diag32.p : nullptr, g->has32 ? d.invd32.p : nullptr);
+    fill_sweeps(g, d);
   }
   const int64_t n0 = g->lv[0].n, nnz0 = h.A[0].nnz();
   k_refresh_vals<<<nblk(nnz0), 256, 0, s>>>(nnz0, a->val.p, g->nat_smap.p, g->nat_v64.p, nullptr);
@@ -2606,6 +2719,24 @@ extern "C" int afe_amg_clone(const afe_amg *src, afe_matrix *a, afe_amg **out) {
     clone_buf(ctx, d.c_val, o.c_val);
     clone_buf(ctx, d.P_val, o.P_val);
     clone_buf(ctx, d.Pt_val, o.Pt_val);
+    for (int k = 0; k < 2; k++) {
+      DevLevel::Sweep &w = d.sweep[k];
+      const DevLevel::Sweep &ow = o.sweep[k];
+      w.nb = ow.nb;
+      w.ncol = ow.ncol;
+      w.gs = ow.gs;
+      w.max_loc = ow.max_loc;
+      w.max_rows = ow.max_rows;
+      w.max_slices = ow.max_slices;
+      w.max_ent = ow.max_ent;
+      clone_buf(ctx, w.blocks, ow.blocks);
+      clone_buf(ctx, w.rows, ow.rows);
+      clone_buf(ctx, w.slices, ow.slices);
+      clone_buf(ctx, w.col_slice, ow.col_slice);
+      clone_buf(ctx, w.cols, ow.cols);
+      clone_buf(ctx, w.src, ow.src);
+    }
+    alloc_sweeps(g.get(), d); // the values come with the refresh below
     d.x64.alloc(ctx, d.n);
     d.b64.alloc(ctx, d.n);
     d.t64.alloc(ctx, d.n);
@@ -2695,6 +2826,8 @@ template <> struct Prec<double> {
   static double *x(DevLevel &d) { return d.x64.p; }
   static double *b(DevLevel &d) { return d.b64.p; }
   static double *t(DevLevel &d) { return d.t64.p; }
+  static double *y(DevLevel &d) { return d.y64.p; }
+  static const double *sv(const DevLevel::Sweep &w) { return w.v64.p; }
   static const LevelDev<double> *ld(afe_amg *g) { return g->ld64.p; }
 };
 template <> struct Prec<float> {
@@ -2706,6 +2839,8 @@ template <> struct Prec<float> {
   static float *x(DevLevel &d) { return d.x32.p; }
   static float *b(DevLevel &d) { return d.b32.p; }
   static float *t(DevLevel &d) { return d.t32.p; }
+  static float *y(DevLevel &d) { return d.y32.p; }
+  static const float *sv(const DevLevel::Sweep &w) { return w.v32.p; }
   static const LevelDev<float> *ld(afe_amg *g) { return g->ld32.p; }
 };
 
@@ -2731,15 +2866,40 @@ template <class T>
 static void issue_vcycle(afe_amg *g, int nu, bool symmetric, hipStream_t st, bool x0_zero) {
   const int Lc = (int)g->lv.size() - 1;
   const bool dense = dense_used(g, nu);
-  const int top = dense ? std::min(g->tail0, g->dense_level) : g->tail0; // levels run as launches
+  // levels run as launches: those before the tail, or all before the dense
+  // level when the ones between have one-launch sweeps (a level of 3692 rows:
+  // two sweeps, residual and transfers 26 us, 50 us in the tail's two legs)
+  int top = dense ? std::min(g->tail0, g->dense_level) : g->tail0;
+  if (dense && nu > 0) {
+    int t = top;
+    while (t < g->dense_level && sweeps_fused<T>(g, g->lv[t])) t++;
+    if (t == g->dense_level) top = t;
+  }
+  const bool to_tail = top < (dense ? g->dense_level : Lc);
+  // one-launch sweeps alternate between the level's x and y: at[l] is the one
+  // that holds the current iterate (x again after the 2 nu sweeps)
+  std::vector<int> at(top, 0);
+  auto fused = [&](DevLevel &d) { return nu > 0 && sweeps_fused<T>(g, d); };
+  auto vec = [&](DevLevel &d, int k) { return k ? Prec<T>::y(d) : Prec<T>::x(d); };
+  auto sweep = [&](DevLevel &d, int &k, bool rev, bool zero, DevLevel *dn) {
+    const DevLevel::Sweep &w = d.sweep[rev ? 1 : 0];
+    const SweepLds lds = sweep_lds_of<T>(w);
+    k_sweep<T><<<w.nb, SWEEP_THREADS, (size_t)lds.total, st>>>(
+        w.blocks.p, w.rows.p, w.slices.p, w.col_slice.p, w.cols.p, Prec<T>::sv(w), w.ncol, w.gs, lds,
+        Prec<T>::invd(d), Prec<T>::b(d), zero ? nullptr : vec(d, k), d.t_si.p, d.t_cols.p, Prec<T>::tv(d),
+        dn ? Prec<T>::x(*dn) : nullptr, vec(d, 1 - k), rev ? 1 : 0);
+    k = 1 - k;
+  };
   for (int l = 0; l < top; l++) {
     DevLevel &d = g->lv[l];
     DevLevel &dn = g->lv[l + 1];
     if (l == 0 && x0_zero && nu == 0) k_fill<T><<<nblk(d.n), 256, 0, st>>>(d.n, Prec<T>::x(d), (T)0);
     // the next level is smoothed by launches from zero: the restriction
     // takes its first colour step
-    const bool first_next = nu > 0 && l + 1 < top;
-    for (int it = 0; it < nu; it++)
+    const bool first_next = nu > 0 && l + 1 < top && !fused(dn);
+    const bool one = fused(d);
+    for (int it = 0; one && it < nu; it++) sweep(d, at[l], false, it == 0 && (l > 0 || x0_zero), nullptr);
+    for (int it = 0; !one && it < nu; it++)
       for (int c = 0; c < d.ncol; c++) {
         if (l == 0 && it == 0 && c == 0 && x0_zero) {
           k_gs_first<T><<<nblk(d.n), 256, 0, st>>>(d.n, d.rows_c0, Prec<T>::b(d), Prec<T>::invd(d), Prec<T>::x(d));
@@ -2752,7 +2912,7 @@ static void issue_vcycle(afe_amg *g, int nu, bool symmetric, hipStream_t st, boo
       k_residual<T, true><<<sblk(d.ns), BLK, 0, st>>>(d.si.p, d.ns, nu > 0 ? d.zs : d.ns, d.cols.p, d.c16.p,
                                                        d.cb16.p, d.cshift,
                                                        Prec<T>::v(d), Prec<T>::diag(d),
-                                                       Prec<T>::b(d), Prec<T>::x(d), Prec<T>::t(d), d.gs,
+                                                       Prec<T>::b(d), vec(d, at[l]), Prec<T>::t(d), d.gs,
                                                        g_tune.xcd);
       k_restrict<T, true><<<sblk(d.p_ns), BLK, 0, st>>>(d.p_si.p, d.p_ns, d.p_cols.p, Prec<T>::pv(d),
                                                          Prec<T>::t(d), Prec<T>::b(dn), Prec<T>::x(dn),
@@ -2762,7 +2922,7 @@ static void issue_vcycle(afe_amg *g, int nu, bool symmetric, hipStream_t st, boo
       k_residual<T, false><<<sblk(d.ns), BLK, 0, st>>>(d.si.p, d.ns, nu > 0 ? d.zs : d.ns, d.cols.p, nullptr,
                                                         nullptr, 0,
                                                         Prec<T>::v(d), Prec<T>::diag(d),
-                                                        Prec<T>::b(d), Prec<T>::x(d), Prec<T>::t(d), d.gs,
+                                                        Prec<T>::b(d), vec(d, at[l]), Prec<T>::t(d), d.gs,
                                                         g_tune.xcd);
       k_restrict<T, false><<<sblk(d.p_ns), BLK, 0, st>>>(d.p_si.p, d.p_ns, d.p_cols.p, Prec<T>::pv(d),
                                                           Prec<T>::t(d), Prec<T>::b(dn), Prec<T>::x(dn),
@@ -2780,10 +2940,10 @@ static void issue_vcycle(afe_amg *g, int nu, bool symmetric, hipStream_t st, boo
     // the levels of the tail above the dense one, its product, and back up
     const int ld = dense ? g->dense_level : Lc;
     DevLevel &dc = g->lv[ld];
-    if (g->tail0 < ld) tail(ld, 1);
+    if (to_tail) tail(ld, 1);
     k_coarse_gemv<T><<<nblk(dc.n, WPB), BLK, 0, st>>>((int)dc.n, dense ? dense_matrix(g, symmetric) : g->minv.p,
                                                        Prec<T>::b(dc), Prec<T>::x(dc));
-    if (g->tail0 < ld) tail(ld, 4);
+    if (to_tail) tail(ld, 4);
   } else {
     tail(Lc, 7);
   }
@@ -2794,6 +2954,10 @@ static void issue_vcycle(afe_amg *g, int nu, bool symmetric, hipStream_t st, boo
     const int lc0 = d.ncol > 0 ? d.colour_row[d.ncol - 1] : (int)d.n;
     const int skip0 = nu == 0 ? 0 : (symmetric ? lc0 : 0);
     const int skip1 = nu == 0 ? 0 : (symmetric ? (int)d.n : (int)d.rows_c0);
+    if (fused(d)) {
+      for (int it = 0; it < nu; it++) sweep(d, at[l], symmetric, false, it == 0 ? &dn : nullptr);
+      continue;
+    }
     if (d.stream)
       k_prolong<T, true><<<sblk(d.t_ns), BLK, 0, st>>>(d.t_si.p, d.t_ns, d.t_cols.p, Prec<T>::tv(d),
                                                         Prec<T>::x(dn), Prec<T>::x(d), skip0, skip1, g_tune.xcd);

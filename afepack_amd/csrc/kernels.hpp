@@ -9,6 +9,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "element_geom.hpp"
@@ -1205,6 +1206,193 @@ __global__ __launch_bounds__(BLK) void k_prolong(const SliceInfo *__restrict__ s
   if (r >= skip0 && r < skip1) return;
   const T xr = x[r];
   x[r] = xr + sell_dot<T, NT, LaunchChunk<T, NT>::v>(q, lane, cols, vals, xc);
+}
+
+// ---------------------------------------------------------------------------
+// a whole colour sweep of a small level in one launch (SweepTables): block k
+// loads x of its local rows (zero without xin; with xc, x + P^T xc, the
+// prolongation), runs the colours on its closure in LDS and writes its own
+// rows to xout, another buffer than xin, from which other blocks still read.
+// What it takes the place of is one launch per colour, each 4 to 5 us of
+// latency for a few thousand rows; the blocks' redundant rows (1.1 to 6 times
+// the level) cost less.  The block's values and columns are staged in LDS, all
+// loads in flight together, so that a colour step waits on LDS and a barrier
+// only.  Latency bound (launch, two or three dependent loads, the colour
+// steps).  FP32, forward / with the prolongation, against the colour launches'
+// 4 us each: 4534 rows of 8 colours 7.9 / 9.2 us, 30230 rows of 6 colours 8.2 /
+// 10.6, 71382 rows of 8 colours 17 / 21.  1024 threads a block, the loads of
+// one block per CU in flight: with 512 threads those take 9.0 / 10.6, 10.8 /
+// 13.6 and 21 / 26 us, with 256 12.7 / 14.0, 13.8 / 15.6 and 31 / 36.
+// ---------------------------------------------------------------------------
+struct SweepLds { // byte offsets of a block's arrays in dynamic LDS
+  int b, d, si, cs, v, c, total;
+};
+template <class T> SweepLds sweep_lds(int max_loc, int max_rows, int max_slices, int ncol, int max_ent) {
+  auto up = [](int64_t o) { return (o + 15) & ~int64_t(15); };
+  int64_t o = up((int64_t)max_loc * sizeof(T));
+  SweepLds l;
+  l.b = (int)o; o = up(o + (int64_t)max_rows * sizeof(T));
+  l.d = (int)o; o = up(o + (int64_t)max_rows * sizeof(T));
+  l.si = (int)o; o = up(o + (int64_t)max_slices * sizeof(SliceInfo));
+  l.cs = (int)o; o = up(o + (int64_t)(ncol + 1) * 4);
+  l.v = (int)o; o = up(o + (int64_t)max_ent * sizeof(T));
+  l.c = (int)o; o = up(o + (int64_t)max_ent * 2);
+  l.total = (int)std::min<int64_t>(o, INT32_MAX);
+  return l;
+}
+
+// nbytes (a multiple of 16) from global memory to LDS, both 16-byte aligned,
+// SWEEP_LOADS loads of 16 bytes in flight per thread
+constexpr int SWEEP_LOADS = 4;
+__device__ __forceinline__ void sweep_stage(void *lds, const void *__restrict__ g, int nbytes, int tid) {
+  const uint4 *src = reinterpret_cast<const uint4 *>(g);
+  uint4 *dst = reinterpret_cast<uint4 *>(lds);
+  const int n = nbytes / 16;
+  for (int i = tid; i < n; i += SWEEP_LOADS * SWEEP_THREADS) {
+    uint4 r[SWEEP_LOADS];
+#pragma unroll
+    for (int u = 0; u < SWEEP_LOADS; u++)
+      if (i + u * SWEEP_THREADS < n) r[u] = src[i + u * SWEEP_THREADS];
+#pragma unroll
+    for (int u = 0; u < SWEEP_LOADS; u++)
+      if (i + u * SWEEP_THREADS < n) dst[i + u * SWEEP_THREADS] = r[u];
+  }
+}
+
+template <class T>
+__global__ __launch_bounds__(SWEEP_THREADS) void k_sweep(
+    const SweepBlock *__restrict__ blocks, const int32_t *__restrict__ rows, const SliceInfo *__restrict__ slices,
+    const int32_t *__restrict__ col_slice, const uint16_t *__restrict__ cols, const T *__restrict__ vals, int ncol,
+    int gs, SweepLds lds, const T *__restrict__ invd, const T *__restrict__ b, const T *__restrict__ xin,
+    const SliceInfo *__restrict__ t_si, const int32_t *__restrict__ t_cols, const T *__restrict__ t_vals,
+    const T *__restrict__ xc, T *__restrict__ xout, int rev) {
+  extern __shared__ __align__(16) char sweep_smem[];
+  T *sx = reinterpret_cast<T *>(sweep_smem);
+  T *sb = reinterpret_cast<T *>(sweep_smem + lds.b);
+  T *sd = reinterpret_cast<T *>(sweep_smem + lds.d);
+  SliceInfo *ssi = reinterpret_cast<SliceInfo *>(sweep_smem + lds.si);
+  int32_t *scs = reinterpret_cast<int32_t *>(sweep_smem + lds.cs);
+  T *sv = reinterpret_cast<T *>(sweep_smem + lds.v);
+  uint16_t *sc = reinterpret_cast<uint16_t *>(sweep_smem + lds.c);
+  const SweepBlock k = blocks[blockIdx.x];
+  const int tid = threadIdx.x;
+  // a block's entries start at a multiple of 64 and are one
+  sweep_stage(sv, vals + k.ent0, k.n_ent * (int)sizeof(T), tid);
+  sweep_stage(sc, cols + k.ent0, k.n_ent * 2, tid);
+  for (int i = tid; i < k.n_slices; i += SWEEP_THREADS) ssi[i] = slices[k.slice0 + i];
+  for (int i = tid; i <= ncol; i += SWEEP_THREADS) scs[i] = col_slice[(int64_t)blockIdx.x * (ncol + 1) + i];
+  for (int i = tid; i < k.n_loc; i += SWEEP_THREADS) {
+    int r = rows[k.row0 + i];
+    if (r < 0) r = ~r;
+    T x = xin ? xin[r] : (T)0;
+    if (xc) { // P^T in one lane per row, 64 rows a slice
+      const SliceInfo q = t_si[r / WAVE];
+      x += sell_dot<T>(q, r % WAVE, t_cols, t_vals, xc);
+    }
+    sx[i] = x;
+    if (i < k.n_rows) {
+      sb[i] = b[r];
+      sd[i] = invd[r];
+    }
+  }
+  __syncthreads();
+  const int lane = tid % WAVE, w = wave_id();
+  const bool lead = (lane & ((1 << gs) - 1)) == 0;
+  auto colour = [&](int step) { return rev ? ncol - 1 - step : step; };
+  // lane t holds what the wavefront needs to know of step t (ncol <= 64): its
+  // first slice there and the colour's slices, so that a step finds them in
+  // registers
+  SliceInfo mine{0, 0, 0, 0};
+  int first = 0, count = 0;
+  if (lane < ncol) {
+    first = scs[colour(lane)];
+    count = scs[colour(lane) + 1] - first;
+    if (w < count) mine = ssi[first + w];
+  }
+  // a wavefront's first slice of a colour: its entries, b and 1/diag, read one
+  // step ahead (none depends on x)
+  constexpr int CH = 4;
+  struct Ahead {
+    int r, width, off;
+    int cc[CH];
+    T vv[CH], br, dr;
+    bool on;
+  };
+  auto issue = [&](Ahead &p, int row0, int nrow, int width, int off) {
+    p.on = (lane >> gs) < nrow;
+    p.r = row0 + (lane >> gs);
+    p.width = width;
+    p.off = off + lane;
+    if (!p.on) return;
+    p.br = sb[p.r];
+    p.dr = sd[p.r];
+#pragma unroll
+    for (int u = 0; u < CH; u++)
+      if (u < width) {
+        p.cc[u] = sc[p.off + u * WAVE];
+        p.vv[u] = sv[p.off + u * WAVE];
+      }
+  };
+  auto finish = [&](const Ahead &p) {
+    if (!p.on) return;
+    T acc = 0, xx[CH];
+#pragma unroll
+    for (int u = 0; u < CH; u++)
+      if (u < p.width) xx[u] = sx[p.cc[u]];
+#pragma unroll
+    for (int u = 0; u < CH; u++)
+      if (u < p.width) acc += p.vv[u] * xx[u];
+    for (int j = CH; j < p.width; j += CH) {
+      int cc[CH];
+      T vv[CH];
+#pragma unroll
+      for (int u = 0; u < CH; u++)
+        if (j + u < p.width) {
+          cc[u] = sc[p.off + (j + u) * WAVE];
+          vv[u] = sv[p.off + (j + u) * WAVE];
+        }
+#pragma unroll
+      for (int u = 0; u < CH; u++)
+        if (j + u < p.width) xx[u] = sx[cc[u]];
+#pragma unroll
+      for (int u = 0; u < CH; u++)
+        if (j + u < p.width) acc += vv[u] * xx[u];
+    }
+    acc = row_group_sum(acc, gs);
+    if (lead) sx[p.r] = (p.br - acc) * p.dr;
+  };
+  auto of_step = [&](int v, int step) { return __builtin_amdgcn_readlane(v, step); };
+  Ahead p;
+  issue(p, of_step(mine.row0, 0), of_step(mine.nrow, 0), of_step(mine.width, 0), of_step(mine.off, 0));
+  for (int step = 0; step < ncol; step++) {
+    finish(p);
+    const int s0 = of_step(first, step), n = of_step(count, step);
+    for (int s = w + SWEEP_THREADS / WAVE; s < n; s += SWEEP_THREADS / WAVE) {
+      Ahead e;
+      const SliceInfo q = ssi[s0 + s];
+      issue(e, q.row0, q.nrow, q.width, q.off);
+      finish(e);
+    }
+    if (step + 1 < ncol)
+      issue(p, of_step(mine.row0, step + 1), of_step(mine.nrow, step + 1), of_step(mine.width, step + 1),
+            of_step(mine.off, step + 1));
+    __syncthreads();
+  }
+  for (int i = tid; i < k.n_rows; i += SWEEP_THREADS) {
+    const int r = rows[k.row0 + i];
+    if (r < 0) xout[~r] = sx[i];
+  }
+}
+
+// the blocks' values from the level's layout (padding: 0)
+__global__ __launch_bounds__(256) void k_sweep_values(int64_t n, const int32_t *__restrict__ src,
+                                                      const double *__restrict__ l64, double *__restrict__ v64,
+                                                      const float *__restrict__ l32, float *__restrict__ v32) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int32_t p = src[i];
+  v64[i] = p < 0 ? 0.0 : l64[p];
+  if (v32) v32[i] = p < 0 ? 0.0f : l32[p];
 }
 
 // ---------------------------------------------------------------------------

@@ -26,7 +26,7 @@ def _pair(ctx, monkeypatch, A, prm, rows):
     return a, afe.Amg(A, prm)
 
 
-def _compare(ctx, g0, g1, n, rng, f32=True):
+def compare(ctx, g0, g1, n, rng, f32=True):
     import afepack_amd as afe
     r = afe.DeviceVector.from_numpy(ctx, rng.uniform(-1, 1, n))
     z = [afe.DeviceVector(ctx, n) for _ in range(2)]
@@ -59,7 +59,7 @@ def test_matrix_form_equals_the_steps(ctx, monkeypatch, kind, n, lazy, smooth, r
     for g in (g0, g1):
         g.set_tail_rows(tail)
     rng = np.random.default_rng(n)
-    _compare(ctx, g0, g1, sp.n_dof, rng)
+    compare(ctx, g0, g1, sp.n_dof, rng)
     xs = []
     for g in (g0, g1):
         x = afe.DeviceVector(ctx, sp.n_dof)
@@ -71,10 +71,10 @@ def test_matrix_form_equals_the_steps(ctx, monkeypatch, kind, n, lazy, smooth, r
         A.apply_dirichlet(b)
         for g in (g0, g1):
             g.lazy_reinit(A)
-        _compare(ctx, g0, g1, sp.n_dof, rng)
+        compare(ctx, g0, g1, sp.n_dof, rng)
     for g in (g0, g1):
         g.set_smooth(2)
-    _compare(ctx, g0, g1, sp.n_dof, rng)
+    compare(ctx, g0, g1, sp.n_dof, rng)
     for g in (g0, g1):
         g.set_coarse_exact(False)
-    _compare(ctx, g0, g1, sp.n_dof, rng)
+    compare(ctx, g0, g1, sp.n_dof, rng)
