@@ -1745,6 +1745,7 @@ struct afe_amg {
   DevBuf<double> wx, wxl, wr, wp, wq, wz, wb, part;
   DevBuf<CgScalars> sc;
   CgScalars *h_sc = nullptr; // pinned
+  double *h_rr = nullptr;    // pinned: the (r, r) partials of a CG iteration (RED_BLOCKS)
   bool has32 = false;
   // captured V-cycles: [precision][symmetric]
   hipGraphExec_t vc_graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
@@ -1777,6 +1778,11 @@ static void drop_graphs(afe_amg *g) {
         (void)hipGraphExecDestroy(e);
         e = nullptr;
       }
+}
+
+static void alloc_pinned(afe_amg *g) {
+  HIPCHK(hipHostMalloc((void **)&g->h_sc, sizeof(CgScalars) + RED_BLOCKS * sizeof(double), hipHostMallocDefault));
+  g->h_rr = reinterpret_cast<double *>(g->h_sc + 1);
 }
 
 static void drop_dense(afe_amg *g) { g->dense[0].nu = g->dense[1].nu = -1; }
@@ -2410,7 +2416,7 @@ extern "C" int afe_amg_create(afe_matrix *a, const afe_amg_params *p, afe_amg **
   const auto t2 = std::chrono::steady_clock::now();
   std::lock_guard<CtxMutex> lk(a->ctx->mu);
   HIPCHK(hipSetDevice(a->ctx->device));
-  HIPCHK(hipHostMalloc((void **)&g->h_sc, sizeof(CgScalars), hipHostMallocDefault));
+  alloc_pinned(g.get());
   upload_layout(g.get(), lay);
   if (verbose()) {
     const auto t3 = std::chrono::steady_clock::now();
@@ -2476,7 +2482,7 @@ extern "C" int afe_amg_destroy(afe_amg *g) {
   (void)hipSetDevice(g->ctx->device);
   (void)hipStreamSynchronize(g->ctx->stream);
   drop_graphs(g);
-  if (g->h_sc) (void)hipHostFree(g->h_sc);
+  if (g->h_sc) (void)hipHostFree(g->h_sc); // h_rr lies in it
   if (g->live0) (void)hipEventDestroy(g->live0);
   if (g->live1) (void)hipEventDestroy(g->live1);
   for (auto &set : g->pev)
@@ -2758,7 +2764,7 @@ extern "C" int afe_amg_clone(const afe_amg *src, afe_matrix *a, afe_amg **out) {
   clone_buf(ctx, g->nat_v64, src->nat_v64);
   clone_buf(ctx, g->nat_diag, src->nat_diag);
   clone_buf(ctx, g->minv, src->minv);
-  HIPCHK(hipHostMalloc((void **)&g->h_sc, sizeof(CgScalars), hipHostMallocDefault));
+  alloc_pinned(g.get());
   finish_levels(g.get());
   device_lazy_refresh(g.get(), a);
   *out = g.release();
@@ -3122,6 +3128,16 @@ extern "C" int afe_amg_precondition(afe_amg *g, double *d_x, const double *d_b, 
   return afe_amg_solve(g, d_x, d_b, 0.0, iterate_step, 1, 0.0, &st);
 }
 
+// blocks of the CG vector kernels (each adds up a kernel's partial sums, so
+// small systems take no more than they need) and of the SpMV
+static unsigned cg_blocks(int64_t n) { return std::min<unsigned>(nblk(n), RED_BLOCKS); }
+static int spmv_grid(const afe_amg *g) {
+  return std::min(g_tune.spmv_blocks, (int)((nblk(g->nat_ns, WPB) + 7) / 8 * 8));
+}
+// up to this many partials of pq are added up by every block of the update
+// (4096: 32 KB a block, 16 loads a thread); more, by a launch of their own
+constexpr int CG_SUM_PARTIALS = 4096;
+
 // z = M^{-1} r with one symmetric V-cycle from zero; r and z in the natural
 // numbering, the V-cycle in the level-0 colour order
 template <class T> static void precondition_perm(afe_amg *g, const double *r, bool first) {
@@ -3131,9 +3147,9 @@ template <class T> static void precondition_perm(afe_amg *g, const double *r, bo
   k_prep_vcycle<T><<<nblk(n), 256, 0, s>>>(n, r, Prec<T>::b(d0), Prec<T>::x(d0), g->iperm0.p);
   launch_graph_or_issue(g, std::is_same<T, float>::value ? 1 : 0, true, g->prm.smooth);
   if (first) k_fill<double><<<nblk(n), 256, 0, s>>>(n, g->wz.p, 0.0);
-  k_take_z<T><<<RED_BLOCKS, 256, 0, s>>>(n, Prec<T>::x(d0), r, g->wz.p, g->iperm0.p, g->part.p);
-  k_finalize_beta<<<1, FIN_THREADS, 0, s>>>(g->part.p, RED_BLOCKS, g->sc.p, first ? 1 : 0);
-  k_p_update<<<RED_BLOCKS, 256, 0, s>>>(n, g->sc.p, g->wz.p, g->wp.p);
+  const unsigned nb = cg_blocks(n);
+  k_take_z<T><<<nb, 256, 0, s>>>(n, Prec<T>::x(d0), r, g->wz.p, g->iperm0.p, g->part.p);
+  k_p_update<<<nb, 256, 0, s>>>(n, g->sc.p, g->part.p, (int)nb, first ? 1 : 0, g->wz.p, g->wp.p);
 }
 
 // one CG iteration after the direction p is set: q = A p, alpha, x/r update,
@@ -3143,31 +3159,40 @@ template <class T> static void precondition_perm(afe_amg *g, const double *r, bo
 // dispatch (hipExtLaunchKernel), so host launch gaps stay out of the figure
 static void issue_cg_spmv(afe_amg *g, hipStream_t s, hipEvent_t start = nullptr, hipEvent_t stop = nullptr) {
   if (start) {
-    hipExtLaunchKernelGGL(k_spmv_dot, dim3(g_tune.spmv_blocks), dim3(BLK), 0, s, start, stop, 0,
+    hipExtLaunchKernelGGL(k_spmv_dot, dim3(spmv_grid(g)), dim3(BLK), 0, s, start, stop, 0,
                           g->nat_si.p, g->nat_ns, g->nat_cols.p, g->nat_c16.p, g->nat_cbase.p, g->nat_v64.p,
                           g->nat_diag.p, g->nat_rowmap.p, g->wp.p, g->wq.p, g->part.p, g_tune.xcd);
     HIPCHK(hipGetLastError());
     return;
   }
-  k_spmv_dot<<<g_tune.spmv_blocks, BLK, 0, s>>>(g->nat_si.p, g->nat_ns, g->nat_cols.p, g->nat_c16.p,
+  k_spmv_dot<<<spmv_grid(g), BLK, 0, s>>>(g->nat_si.p, g->nat_ns, g->nat_cols.p, g->nat_c16.p,
                                                  g->nat_cbase.p, g->nat_v64.p, g->nat_diag.p, g->nat_rowmap.p,
                                                  g->wp.p, g->wq.p, g->part.p, g_tune.xcd);
 }
 
 // part 0 of a CG iteration after the SpMV: alpha, the x / r update with the
-// FP32 (or FP64) right-hand side of the V-cycle, (r, r), and the scalars to
-// the host
+// FP32 (or FP64) right-hand side of the V-cycle, and the partials of (r, r) to
+// the host.  The sums of partials that a kernel needs are taken by its blocks,
+// not by launches between: four CG launches an iteration, not seven (263K P2
+// DOFs 174 -> 167 us an iteration, 4.2M 804 -> 798)
 template <class T> static void issue_cg_update(afe_amg *g) {
   DevLevel &d0 = g->lv[0];
   hipStream_t s = g->ctx->stream;
   const int64_t n = d0.n;
-  k_finalize<<<1, FIN_THREADS, 0, s>>>(g->part.p, g_tune.spmv_blocks, 1, &g->sc.p->pq);
+  const int np = spmv_grid(g);
+  if (np > CG_SUM_PARTIALS) k_finalize<<<1, FIN_THREADS, 0, s>>>(g->part.p, np, 1, &g->sc.p->pq);
   // level 0 runs as launches (tail0 > 0): the V-cycle's first colour kernel
   // sets x0, so the update does not clear it
-  k_cg_update<T><<<RED_BLOCKS, 256, 0, s>>>(n, g->sc.p, g->wx.p, g->wxl.p, g->wr.p, g->wp.p, g->wq.p,
-                                             Prec<T>::b(d0), g->tail0 > 0 ? nullptr : Prec<T>::x(d0),
-                                             g->iperm0.p, g->part.p);
-  k_finalize_host<<<1, FIN_THREADS, 0, s>>>(g->part.p, RED_BLOCKS, &g->sc.p->rr, g->sc.p, g->h_sc);
+  k_cg_update<T><<<cg_blocks(n), 256, 0, s>>>(n, g->sc.p, g->part.p, np > CG_SUM_PARTIALS ? 0 : np, g->wx.p,
+                                               g->wxl.p, g->wr.p, g->wp.p, g->wq.p, Prec<T>::b(d0),
+                                               g->tail0 > 0 ? nullptr : Prec<T>::x(d0), g->iperm0.p, g->h_rr);
+}
+
+// (r, r) of the iteration whose part 0 has completed, in block order
+static double cg_rr(const afe_amg *g) {
+  double rr = 0.0;
+  for (unsigned k = 0; k < cg_blocks(g->lv[0].n); k++) rr += g->h_rr[k];
+  return rr;
 }
 
 // part 1: z = M r (the V-cycle, issued inline: nested capture is not used),
@@ -3177,9 +3202,9 @@ template <class T> static void issue_cg_precondition(afe_amg *g) {
   hipStream_t s = g->ctx->stream;
   const int64_t n = d0.n;
   issue_vcycle<T>(g, g->prm.smooth, true, s, true);
-  k_take_z<T><<<RED_BLOCKS, 256, 0, s>>>(n, Prec<T>::x(d0), g->wr.p, g->wz.p, g->iperm0.p, g->part.p);
-  k_finalize_beta<<<1, FIN_THREADS, 0, s>>>(g->part.p, RED_BLOCKS, g->sc.p, 0);
-  k_p_update<<<RED_BLOCKS, 256, 0, s>>>(n, g->sc.p, g->wz.p, g->wp.p);
+  const unsigned nb = cg_blocks(n);
+  k_take_z<T><<<nb, 256, 0, s>>>(n, Prec<T>::x(d0), g->wr.p, g->wz.p, g->iperm0.p, g->part.p);
+  k_p_update<<<nb, 256, 0, s>>>(n, g->sc.p, g->part.p, (int)nb, 0, g->wz.p, g->wp.p);
 }
 
 // launches one captured part (capturing it on first use or after a change
@@ -3295,10 +3320,8 @@ static int pcg_impl(afe_amg *g, double *d_x, const double *d_b, double rtol, int
         }
       }
       it++;
-      rr = g->h_sc->rr;
-      if (verbose())
-        fprintf(stderr, "pcg it %d rel res %.3e pq %.3e rz %.3e beta %.3e\n", it, std::sqrt(rr / bb),
-                g->h_sc->pq, g->h_sc->rz, g->h_sc->beta);
+      rr = cg_rr(g);
+      if (verbose()) fprintf(stderr, "pcg it %d rel res %.3e\n", it, std::sqrt(rr / bb));
       if (!(rr == rr)) {
         HIPCHK(hipStreamSynchronize(s)); // part 1 of the iteration is still queued
         g->part_pending = false;

@@ -2157,29 +2157,18 @@ struct CgScalars {
   double rz, pq, rz_new, rz_cross, rr, bb, l1, beta;
 };
 
-// k_finalize of one sum into *out (a field of *sc), then the scalars copied
-// to pinned host memory by the thread that wrote the sum, so the host reads
-// them once the launch is complete without a separate copy (vector stores
-// to host-coherent memory; the launch's completion makes them visible)
-__global__ __launch_bounds__(FIN_THREADS) void k_finalize_host(const double *__restrict__ part, int np,
-                                                               double *out, const CgScalars *sc,
-                                                               CgScalars *__restrict__ h_sc) {
-  __shared__ double sh[FIN_THREADS];
-  double s = strided_sum(part, np, threadIdx.x, blockDim.x);
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) {
-    *out = s;
-    const CgScalars v = *sc;
-    *h_sc = v;
-  }
-}
-
 #pragma clang fp contract(off)
 // alpha = rz / pq; x += alpha p kept as the unevaluated pair x_hi + x_lo
 // (the sum and the product errors go to x_lo); r -= alpha q;
-// (T) r -> b0, x0 = 0; partial (r, r)
+// (T) r -> b0, x0 = 0; partial (r, r).
+// With np > 0 every block adds up the np partials of pq itself (all in the
+// same order, the same bits), which saves the launch between the SpMV and the
+// update; np = 0 takes the finalized sc->pq.  The partials of (r, r) go to
+// pinned host memory: the host adds them up.  sc->rz_new is the rz of the last
+// preconditioning; block 0 moves it to sc->rz, which no block reads here.
 template <class T>
-__global__ __launch_bounds__(256) void k_cg_update(int64_t n, const CgScalars *__restrict__ sc,
+__global__ __launch_bounds__(256) void k_cg_update(int64_t n, CgScalars *__restrict__ sc,
+                                                   const double *__restrict__ pq_part, int np,
                                                    double *__restrict__ x, double *__restrict__ xl,
                                                    double *__restrict__ r,
                                                    const double *__restrict__ p, const double *__restrict__ q,
@@ -2187,7 +2176,10 @@ __global__ __launch_bounds__(256) void k_cg_update(int64_t n, const CgScalars *_
                                                    const int32_t *__restrict__ iperm,
                                                    double *__restrict__ part) {
   __shared__ double sh[256];
-  const double alpha = sc->rz / sc->pq;
+  const double rz = sc->rz_new;
+  const double pq = np > 0 ? block_sum(strided_sum(pq_part, np, threadIdx.x, blockDim.x), sh) : sc->pq;
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc->rz = rz;
+  const double alpha = rz / pq;
   double rr = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -2270,26 +2262,20 @@ __global__ __launch_bounds__(256) void k_take_z(int64_t n, const T *__restrict__
   }
 }
 
-// k_finalize of the (r, z_new) and (r, z_old) partials into rz_new and
-// rz_cross, then (the same thread, in order) the flexible (Polak-Ribiere)
-// beta = (rz_new - rz_cross) / rz, robust to the FP32 preconditioner
-// (first != 0: beta = 0, p = z), and rz = rz_new
-__global__ __launch_bounds__(FIN_THREADS) void k_finalize_beta(const double *__restrict__ part, int np,
-                                                               CgScalars *__restrict__ sc, int first) {
-  __shared__ double sh[FIN_THREADS];
-  double v[2];
-  for (int k = 0; k < 2; k++) v[k] = block_sum(strided_sum(part + (int64_t)k * np, np, threadIdx.x, blockDim.x), sh);
-  if (threadIdx.x == 0) {
-    sc->rz_new = v[0];
-    sc->rz_cross = v[1];
-    sc->beta = first ? 0.0 : (v[0] - v[1]) / sc->rz;
-    sc->rz = v[0];
-  }
-}
-
-__global__ __launch_bounds__(256) void k_p_update(int64_t n, const CgScalars *__restrict__ sc,
+// p = z + beta p with the flexible (Polak-Ribiere) beta = (rz_new - rz_cross)
+// / rz, robust to the FP32 preconditioner (first != 0: beta = 0, p = z).
+// Every block adds up the np partials of rz_new and of rz_cross itself (the
+// same order, the same bits), which saves a launch; block 0 stores rz_new,
+// which no block reads here.
+__global__ __launch_bounds__(256) void k_p_update(int64_t n, CgScalars *__restrict__ sc,
+                                                  const double *__restrict__ part, int np, int first,
                                                   const double *__restrict__ z, double *__restrict__ p) {
-  const double beta = sc->beta;
+  __shared__ double sh[256];
+  const double rz = sc->rz;
+  const double rz_new = block_sum(strided_sum(part, np, threadIdx.x, blockDim.x), sh);
+  const double cross = block_sum(strided_sum(part + np, np, threadIdx.x, blockDim.x), sh);
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc->rz_new = rz_new;
+  const double beta = first ? 0.0 : (rz_new - cross) / rz;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
     p[i] = z[i] + beta * p[i];
