@@ -1665,13 +1665,16 @@ struct DevLevel {
   struct Sweep {
     int nb = 0, ncol = 0, gs = 0;
     int max_loc = 0, max_rows = 0, max_slices = 0, max_ent = 0;
-    DevBuf<SweepBlock> blocks;
-    DevBuf<int32_t> rows, col_slice, src;
-    DevBuf<SliceInfo> slices;
-    DevBuf<uint16_t> cols;
-    DevBuf<double> v64;
-    DevBuf<float> v32;
+    int64_t n_ent = 0;  // entries of all blocks
+    int64_t val0 = 0;   // the direction's first value in sweep_v64 / sweep_v32
+    int64_t blocks = 0, rows = 0, slices = 0, col_slice = 0, cols = 0, src = 0; // byte offsets in sweep_tab
   } sweep[2];
+  // both directions' tables in one buffer, their values in one per precision
+  // (a few dozen buffers of their own took longer to set up than to fill)
+  DevBuf<char> sweep_tab;
+  DevBuf<double> sweep_v64;
+  DevBuf<float> sweep_v32;
+  template <class U> const U *tab(int64_t off) const { return reinterpret_cast<const U *>(sweep_tab.p + off); }
   DevBuf<double> y64;
   DevBuf<float> y32;
   std::vector<int32_t> perm; // new -> old
@@ -2167,14 +2170,13 @@ static void ensure_dense(afe_amg *g, bool symmetric, int nu) {
 
 // the blocks' value arrays and the second level vector
 static void alloc_sweeps(afe_amg *g, DevLevel &d) {
-  for (DevLevel::Sweep &w : d.sweep) {
-    if (w.nb == 0) continue;
-    w.v64.alloc(g->ctx, w.src.n);
-    d.y64.alloc(g->ctx, d.n);
-    if (g->has32) {
-      w.v32.alloc(g->ctx, w.src.n);
-      d.y32.alloc(g->ctx, d.n);
-    }
+  if (d.sweep[0].nb == 0) return;
+  const size_t n = (size_t)(d.sweep[0].n_ent + d.sweep[1].n_ent);
+  d.sweep_v64.alloc(g->ctx, n);
+  d.y64.alloc(g->ctx, d.n);
+  if (g->has32) {
+    d.sweep_v32.alloc(g->ctx, n);
+    d.y32.alloc(g->ctx, d.n);
   }
 }
 
@@ -2182,8 +2184,9 @@ static void alloc_sweeps(afe_amg *g, DevLevel &d) {
 static void fill_sweeps(afe_amg *g, DevLevel &d) {
   for (DevLevel::Sweep &w : d.sweep)
     if (w.nb > 0)
-      k_sweep_values<<<nblk(w.src.n), 256, 0, g->ctx->stream>>>((int64_t)w.src.n, w.src.p, d.v64.p, w.v64.p, d.v32.p,
-                                                                w.v32.p);
+      k_sweep_values<<<nblk(w.n_ent), 256, 0, g->ctx->stream>>>(
+          w.n_ent, d.tab<int32_t>(w.src), d.v64.p, d.sweep_v64.p + w.val0, d.v32.p,
+          g->has32 ? d.sweep_v32.p + w.val0 : nullptr);
   HIPCHK(hipGetLastError());
 }
 
@@ -2251,6 +2254,8 @@ static void upload_layout(afe_amg *g, HostLayout &lay) {
         d.t_v32.upload(ctx, to_prec<float>(st.vals));
       }
     }
+    std::vector<char> tab;
+    int64_t val0 = 0;
     for (int k = 0; k < 2; k++) {
       const SweepTables &t = hl.sweep[k];
       DevLevel::Sweep &w = d.sweep[k];
@@ -2262,12 +2267,26 @@ static void upload_layout(afe_amg *g, HostLayout &lay) {
       w.max_rows = t.max_rows;
       w.max_slices = t.max_slices;
       w.max_ent = t.max_ent;
-      w.blocks.upload(ctx, t.blocks);
-      w.rows.upload(ctx, t.rows);
-      w.slices.upload(ctx, t.slices);
-      w.col_slice.upload(ctx, t.col_slice);
-      w.cols.upload(ctx, t.cols);
-      w.src.upload(ctx, t.src);
+      w.n_ent = (int64_t)t.src.size();
+      w.val0 = val0;
+      val0 += w.n_ent;
+      auto put = [&](const auto &v) {
+        const int64_t off = (int64_t)(tab.size() + 255) / 256 * 256;
+        const char *p = reinterpret_cast<const char *>(v.data());
+        tab.resize(off);
+        tab.insert(tab.end(), p, p + v.size() * sizeof(v[0]));
+        return off;
+      };
+      w.blocks = put(t.blocks);
+      w.rows = put(t.rows);
+      w.slices = put(t.slices);
+      w.col_slice = put(t.col_slice);
+      w.cols = put(t.cols);
+      w.src = put(t.src);
+    }
+    if (!tab.empty()) {
+      d.sweep_tab.upload(ctx, tab);
+      HIPCHK(hipStreamSynchronize(ctx->stream)); // tab goes out of scope
     }
     alloc_sweeps(g, d);
     d.x64.alloc(ctx, d.n);
@@ -2725,23 +2744,8 @@ extern "C" int afe_amg_clone(const afe_amg *src, afe_matrix *a, afe_amg **out) {
     clone_buf(ctx, d.c_val, o.c_val);
     clone_buf(ctx, d.P_val, o.P_val);
     clone_buf(ctx, d.Pt_val, o.Pt_val);
-    for (int k = 0; k < 2; k++) {
-      DevLevel::Sweep &w = d.sweep[k];
-      const DevLevel::Sweep &ow = o.sweep[k];
-      w.nb = ow.nb;
-      w.ncol = ow.ncol;
-      w.gs = ow.gs;
-      w.max_loc = ow.max_loc;
-      w.max_rows = ow.max_rows;
-      w.max_slices = ow.max_slices;
-      w.max_ent = ow.max_ent;
-      clone_buf(ctx, w.blocks, ow.blocks);
-      clone_buf(ctx, w.rows, ow.rows);
-      clone_buf(ctx, w.slices, ow.slices);
-      clone_buf(ctx, w.col_slice, ow.col_slice);
-      clone_buf(ctx, w.cols, ow.cols);
-      clone_buf(ctx, w.src, ow.src);
-    }
+    for (int k = 0; k < 2; k++) d.sweep[k] = o.sweep[k];
+    clone_buf(ctx, d.sweep_tab, o.sweep_tab);
     alloc_sweeps(g.get(), d); // the values come with the refresh below
     d.x64.alloc(ctx, d.n);
     d.b64.alloc(ctx, d.n);
@@ -2833,7 +2837,7 @@ template <> struct Prec<double> {
   static double *b(DevLevel &d) { return d.b64.p; }
   static double *t(DevLevel &d) { return d.t64.p; }
   static double *y(DevLevel &d) { return d.y64.p; }
-  static const double *sv(const DevLevel::Sweep &w) { return w.v64.p; }
+  static const double *sv(const DevLevel &d) { return d.sweep_v64.p; }
   static const LevelDev<double> *ld(afe_amg *g) { return g->ld64.p; }
 };
 template <> struct Prec<float> {
@@ -2846,7 +2850,7 @@ template <> struct Prec<float> {
   static float *b(DevLevel &d) { return d.b32.p; }
   static float *t(DevLevel &d) { return d.t32.p; }
   static float *y(DevLevel &d) { return d.y32.p; }
-  static const float *sv(const DevLevel::Sweep &w) { return w.v32.p; }
+  static const float *sv(const DevLevel &d) { return d.sweep_v32.p; }
   static const LevelDev<float> *ld(afe_amg *g) { return g->ld32.p; }
 };
 
@@ -2891,7 +2895,8 @@ static void issue_vcycle(afe_amg *g, int nu, bool symmetric, hipStream_t st, boo
     const DevLevel::Sweep &w = d.sweep[rev ? 1 : 0];
     const SweepLds lds = sweep_lds_of<T>(w);
     k_sweep<T><<<w.nb, SWEEP_THREADS, (size_t)lds.total, st>>>(
-        w.blocks.p, w.rows.p, w.slices.p, w.col_slice.p, w.cols.p, Prec<T>::sv(w), w.ncol, w.gs, lds,
+        d.tab<SweepBlock>(w.blocks), d.tab<int32_t>(w.rows), d.tab<SliceInfo>(w.slices),
+        d.tab<int32_t>(w.col_slice), d.tab<uint16_t>(w.cols), Prec<T>::sv(d) + w.val0, w.ncol, w.gs, lds,
         Prec<T>::invd(d), Prec<T>::b(d), zero ? nullptr : vec(d, k), d.t_si.p, d.t_cols.p, Prec<T>::tv(d),
         dn ? Prec<T>::x(*dn) : nullptr, vec(d, 1 - k), rev ? 1 : 0);
     k = 1 - k;
