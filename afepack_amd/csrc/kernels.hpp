@@ -1244,12 +1244,13 @@ template <class T> SweepLds sweep_lds(int max_loc, int max_rows, int max_slices,
 // nbytes (a multiple of 16) from global memory to LDS, both 16-byte aligned,
 // SWEEP_LOADS loads of 16 bytes in flight per thread
 constexpr int SWEEP_LOADS = 4;
+typedef int sweep_vec __attribute__((ext_vector_type(4))); // (a uint4 array went through scratch memory)
 __device__ __forceinline__ void sweep_stage(void *lds, const void *__restrict__ g, int nbytes, int tid) {
-  const uint4 *src = reinterpret_cast<const uint4 *>(g);
-  uint4 *dst = reinterpret_cast<uint4 *>(lds);
+  const sweep_vec *src = reinterpret_cast<const sweep_vec *>(g);
+  sweep_vec *dst = reinterpret_cast<sweep_vec *>(lds);
   const int n = nbytes / 16;
   for (int i = tid; i < n; i += SWEEP_LOADS * SWEEP_THREADS) {
-    uint4 r[SWEEP_LOADS];
+    sweep_vec r[SWEEP_LOADS];
 #pragma unroll
     for (int u = 0; u < SWEEP_LOADS; u++)
       if (i + u * SWEEP_THREADS < n) r[u] = src[i + u * SWEEP_THREADS];
