@@ -988,20 +988,21 @@ static void launch_gather(afe_matrix *a, int64_t b0, int64_t b1, hipStream_t st)
 
 static void launch_gather(afe_matrix *a) { launch_gather(a, 0, gather_blocks(a->s), a->ctx->stream); }
 
-// number of element chunks of a pipelined assembly: 8 for tetrahedral
-// meshes from 2^18 elements up, where the gather (rows of ~24 elements) is
-// latency bound and leaves the chip room for the next chunk's element
-// matrices (C3, variable coefficient: 5.3 -> 4.0 ms; constant: no change);
-// 1 (no pipeline) on triangles, where the gather streams at bandwidth and
-// the overlap measured slower (C2 0.50 -> 0.53 ms, P2 variable coefficient
-// 1.37 -> 1.63 ms).  AFE_ASM_CHUNKS=k forces k chunks.
-static int asm_chunks(int kind, int64_t n_elem) {
+// number of element chunks of a pipelined assembly: 8 for the variable
+// coefficient on 6M tetrahedra and more, else 1 (no pipeline).  Each chunk's
+// cross-stream waits cost 15 to 40 us, which the overlap has to earn: 12.6M
+// tetrahedra, 16 modes, 1.82 -> 1.56 ms; 3.1M 0.51 ms whole and 0.60 in 8 chunks;
+// 0.38M 97 and 404 us.  Where the element matrices are short the gather is left
+// nothing to overlap with: constant coefficient, 12.6M, 1.30 whole and 1.48 ms.
+// On triangles the gather streams at bandwidth (2.1M P2 elements 0.50 and 0.53 ms).
+// AFE_ASM_CHUNKS=k forces k chunks.
+static int asm_chunks(int kind, int op, int64_t n_elem) {
   static const int forced = [] {
     const char *e = getenv("AFE_ASM_CHUNKS");
     return e ? std::max(1, std::min(kAsmChunksMax, atoi(e))) : 0;
   }();
   if (forced) return forced;
-  return kind == P1_TET && n_elem >= (int64_t(1) << 18) ? 8 : 1;
+  return kind == P1_TET && op == AFE_OP_VARSTIFF && n_elem >= 6000000 ? 8 : 1;
 }
 
 // Element matrices and CSR gather of afe_assemble.  Pipelined: the elements
@@ -1015,7 +1016,7 @@ static void launch_assembly(afe_matrix *a, int op, const QuadRule *q, FieldDev f
   afe_space *s = a->s;
   afe_ctx *c = a->ctx;
   const int64_t ne = s->h.n_elem, nb = gather_blocks(s);
-  const int K = (int64_t)s->gather_dep.size() == nb ? asm_chunks(s->h.kind, ne) : 1;
+  const int K = (int64_t)s->gather_dep.size() == nb ? asm_chunks(s->h.kind, op, ne) : 1;
   if (K <= 1) {
     launch_elements(a, op, q, fd, 0, ne, c->stream);
     launch_gather(a, 0, nb, c->stream);
