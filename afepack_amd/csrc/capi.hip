@@ -2127,45 +2127,62 @@ static const double *dense_matrix(const afe_amg *g, bool symmetric) {
   return g->dense_level == (int)g->lv.size() - 1 ? g->minv.p : g->dense[symmetric ? 1 : 0].m.p;
 }
 
-// builds the matrix of the sub-cycle if it is used and not current: one
-// workgroup per column runs the tail's FP64 cycle on a unit vector
-static void ensure_dense(afe_amg *g, bool symmetric, int nu) {
-  const int ld = g->dense_level, L = (int)g->lv.size(), nl = L - ld;
-  if (!dense_used(g, nu) || ld == L - 1) return;
-  afe_amg::Dense &d = g->dense[symmetric ? 1 : 0];
-  if (d.nu == nu) return;
+// the matrix of the sub-cycle from level ld to level lc, whose coarse solve
+// is (minv, coarse_mode): one workgroup per column runs the tail's FP64 cycle
+// on a unit vector; throws when there is no memory for it
+static void build_dense(afe_amg *g, int ld, int lc, const double *minv, int coarse_mode, bool symmetric, int nu,
+                        DevBuf<double> &out) {
   afe_ctx *ctx = g->ctx;
   hipStream_t st = ctx->stream;
-  const int n = (int)g->lv[ld].n;
+  const int n = (int)g->lv[ld].n, nl = lc - ld + 1;
   int64_t stride = 0;
-  for (int l = ld; l < L; l++) stride += 3 * g->lv[l].n;
+  for (int l = ld; l <= lc; l++) stride += 3 * g->lv[l].n;
   // columns at a time: at most 256 MB of vectors
   const int cols = (int)std::min<int64_t>(n, std::max<int64_t>(256, (int64_t(32) << 20) / stride));
   DevBuf<LevelDev<double>> tl;
   DevBuf<TailJob<double>> jobs;
   DevBuf<double> own;
-  double *W;
+  out.alloc(ctx, (size_t)n * n);
+  tl.alloc(ctx, (size_t)cols * nl);
+  jobs.alloc(ctx, cols);
+  double *W = call_scratch(ctx, (size_t)cols * stride, own);
+  const int lds_cap = (int)ctx->lds_bytes;
+  for (int c0 = 0; c0 < n; c0 += cols) {
+    const int m = std::min(cols, n - c0);
+    k_fill<double><<<nblk(m * stride), 256, 0, st>>>(m * stride, W, 0.0);
+    k_dense_columns<<<nblk(m), 256, 0, st>>>(m, c0, nl, g->ld64.p + ld, stride, W, tl.p, jobs.p, minv, coarse_mode);
+    kb_tail<double><<<m, TAIL_THREADS, (size_t)lds_cap, st>>>(jobs.p, tl.p, nu, symmetric ? 1 : 0, lds_cap);
+    k_dense_store<<<dim3(nblk(n, 32), nblk(m, 32)), 256, 0, st>>>(n, m, c0, stride, W, out.p);
+  }
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(st)); // before the tables go
+}
+
+// builds the matrix of the sub-cycle if it is used and not current.  In two
+// steps when a level of at most COARSE_TAIL_MAX rows lies further down: that
+// level's matrix first, in one round of workgroups, which then is the coarse
+// solve of all the other columns (2213 rows with levels of 692, 227, 81 and 33
+// below, V(3,3): the first solve on new values 6.0 -> 3.6 ms).
+static void ensure_dense(afe_amg *g, bool symmetric, int nu) {
+  const int ld = g->dense_level, Lc = (int)g->lv.size() - 1;
+  if (!dense_used(g, nu) || ld == Lc) return;
+  afe_amg::Dense &d = g->dense[symmetric ? 1 : 0];
+  if (d.nu == nu) return;
   try {
-    d.m.alloc(ctx, (size_t)n * n);
-    tl.alloc(ctx, (size_t)cols * nl);
-    jobs.alloc(ctx, cols);
-    W = call_scratch(ctx, (size_t)cols * stride, own);
+    int lc = ld + 1;
+    while (lc < Lc && g->lv[lc].n > COARSE_TAIL_MAX) lc++;
+    if (lc < Lc) {
+      DevBuf<double> inner;
+      build_dense(g, lc, Lc, g->minv.p, g->coarse_mode, symmetric, nu, inner);
+      build_dense(g, ld, lc, inner.p, 0, symmetric, nu, d.m);
+    } else {
+      build_dense(g, ld, Lc, g->minv.p, g->coarse_mode, symmetric, nu, d.m);
+    }
   } catch (const afe::Error &) { // no room: the levels stay as they are
     g->dense_off = true;
     drop_graphs(g);
     return;
   }
-  const int lds_cap = (int)ctx->lds_bytes;
-  for (int c0 = 0; c0 < n; c0 += cols) {
-    const int m = std::min(cols, n - c0);
-    k_fill<double><<<nblk(m * stride), 256, 0, st>>>(m * stride, W, 0.0);
-    k_dense_columns<<<nblk(m), 256, 0, st>>>(m, c0, nl, g->ld64.p + ld, stride, W, tl.p, jobs.p, g->minv.p,
-                                             g->coarse_mode);
-    kb_tail<double><<<m, TAIL_THREADS, (size_t)lds_cap, st>>>(jobs.p, tl.p, nu, symmetric ? 1 : 0, lds_cap);
-    k_dense_store<<<dim3(nblk(n, 32), nblk(m, 32)), 256, 0, st>>>(n, m, c0, stride, W, d.m.p);
-  }
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(st)); // before the tables go
   d.nu = nu;
 }
 

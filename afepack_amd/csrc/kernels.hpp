@@ -1728,25 +1728,27 @@ __device__ __forceinline__ void tail_body(const LevelDev<T> *__restrict__ L, int
   if (phase & 2) {
     const LevelDev<T> &d = L[lc];
     if (coarse_mode == 0) {
+      // a wavefront per row, four rows at a time: coalesced row reads, the
+      // lanes' sums added over lane distance 32, 16, ... 1
       const GPtr<const T> b = gptr((const T *)d.b);
       const GPtr<T> x = gptr(d.x);
-      for (int i = tid; i < d.n; i += blockDim.x) {
-        const GPtr<const double> m = gptr(minv) + (int64_t)i * d.n;
-        double s = 0.0;
-        for (int j0 = 0; j0 < d.n; j0 += 8) { // 8 loads in flight, summed in order
-          double mm[8];
-          T bb[8];
+      constexpr int U = 4;
+      for (int i0 = w; i0 < d.n; i0 += U * nw) {
+        double s[U] = {0.0, 0.0, 0.0, 0.0};
+        for (int j = lane; j < d.n; j += WAVE) {
+          const double bj = (double)b[j];
+          double m[U];
 #pragma unroll
-          for (int k = 0; k < 8; k++)
-            if (j0 + k < d.n) {
-              mm[k] = m[j0 + k];
-              bb[k] = b[j0 + k];
-            }
+          for (int u = 0; u < U; u++) m[u] = i0 + u * nw < d.n ? gptr(minv)[(int64_t)(i0 + u * nw) * d.n + j] : 0.0;
 #pragma unroll
-          for (int k = 0; k < 8; k++)
-            if (j0 + k < d.n) s += mm[k] * (double)bb[k];
+          for (int u = 0; u < U; u++) s[u] += m[u] * bj;
         }
-        x[i] = (T)s;
+#pragma unroll
+        for (int o = WAVE / 2; o > 0; o >>= 1)
+#pragma unroll
+          for (int u = 0; u < U; u++) s[u] += __shfl_xor(s[u], o, WAVE);
+        if (lane < U && i0 + lane * nw < d.n)
+          x[i0 + lane * nw] = (T)(lane == 0 ? s[0] : lane == 1 ? s[1] : lane == 2 ? s[2] : s[3]);
       }
     } else if (coarse_mode == 1) {
       for (int i = tid; i < d.n; i += blockDim.x) gptr(d.x)[i] = gptr(d.b)[i] * gptr(d.invd)[i];
