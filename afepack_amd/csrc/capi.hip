@@ -1891,12 +1891,15 @@ static void colour_code(HostLevel &hl) {
 // ones fill the chip with each colour and are bandwidth bound: with the bound at
 // 40K / 131K / 300K rows the CG of 263K P2 DOFs takes 9.02 / 9.03 / 9.66 ms,
 // the moving-mesh step of 251K P1 DOFs 6.78 / 6.65 / 6.86, the CG of 4.2M P2
-// DOFs 49.0 / 48.6 / 48.6 and 53.7 with its 481K-row level), of rows of at most SWEEP_ROW_ENTRIES entries on average and with
-// closures of at most SWEEP_FACTOR times the level (the Galerkin levels of
+// DOFs 49.0 / 48.6 / 48.6 and 53.7 with its 481K-row level), of rows of at most
+// SWEEP_ROW_ENTRIES entries on average and with closures of at most
+// SWEEP_FACTOR times the level (the Galerkin levels of
 // tetrahedra couple 40 rows and more: a block's closure there is a large part
 // of the level).  Levels inside the dense sub-cycle need none, nor do the
 // server's hierarchies, which its batch runs with shared launches.
-// AFE_SWEEP_ROWS sets the bound for hierarchies built afterwards (0: none).
+// The tables cost set-up time: 16 hierarchies of 2K to 214K rows 504 -> 605 ms
+// (582 with 40K).  AFE_SWEEP_ROWS sets the bound for hierarchies built
+// afterwards (0: none).
 constexpr int64_t SWEEP_ROWS = 131072, SWEEP_ROW_ENTRIES = 24, SWEEP_BLOCK_MIN = 32, SWEEP_BLOCK_MAX = 320;
 constexpr double SWEEP_FACTOR = 6.0;
 static int64_t dense_rows_bound();

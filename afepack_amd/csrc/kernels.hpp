@@ -2180,8 +2180,8 @@ __global__ __launch_bounds__(256) void k_dd_round(int64_t n, double *__restrict_
 }
 #pragma clang fp contract(on)
 
-// device scalars of the CG loop; k_finalize writes consecutive fields
-// (rz_new, rz_cross) and (rr, bb, l1) in one call
+// device scalars of the CG loop; k_finalize writes the consecutive fields
+// (rr, bb, l1) in one call
 struct CgScalars {
   double rz, pq, rz_new, rz_cross, rr, bb, l1, beta;
 };
