@@ -558,6 +558,16 @@ class Amg(_AmgBase):
                         "row_lanes": g.value})
         return out
 
+    def sweep_info(self):
+        """per level: blocks of the one-launch sweeps (0: none), rows they update (forward, reverse), fused in
+        (FP64, FP32)"""
+        out = []
+        for l in range(self.info()["levels"]):
+            b, u, f = C.c_int32(), (C.c_int64 * 2)(), (C.c_int32 * 2)()
+            _chk(_lib().afe_amg_sweep_info(self.h, l, C.byref(b), u, f))
+            out.append({"blocks": b.value, "updated": tuple(u), "fused": tuple(bool(v) for v in f)})
+        return out
+
 
 class Batch:
     """Continuous batching of FP64 CG solves preconditioned by one V-cycle

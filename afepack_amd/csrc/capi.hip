@@ -346,6 +346,9 @@ extern "C" int afe_ctx_create(int device, afe_ctx **out) {
                                (int)c->lds_bytes));
     HIPCHK(hipFuncSetAttribute((const void *)k_sweep<double>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)c->lds_bytes));
+    const void *tables[] = {(const void *)k_sweep_closure, (const void *)k_sweep_rows, (const void *)k_sweep_entries};
+    for (const void *f : tables)
+      HIPCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(c->lds_bytes - SWEEP_TABLE_LDS)));
     for (const void *f : staged)
       HIPCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->lds_bytes));
   }
@@ -1661,23 +1664,23 @@ struct DevLevel {
   DevBuf<double> x64, b64, t64;
   DevBuf<float> x32, b32, t32;
   // whole sweeps as one launch (k_sweep): forward [0] and reverse [1]; nb = 0
-  // when the level runs one launch per colour.  y32 / y64: the second vector
-  // that the sweeps write while they read x, and the other way round
+  // when the level runs one launch per colour, or its tables are not formed yet
+  bool sweep_may = false; // the level's size and rows allow them
   struct Sweep {
-    int nb = 0, ncol = 0, gs = 0;
-    int max_loc = 0, max_rows = 0, max_slices = 0, max_ent = 0;
-    int64_t n_ent = 0;  // entries of all blocks
-    int64_t val0 = 0;   // the direction's first value in sweep_v64 / sweep_v32
-    int64_t blocks = 0, rows = 0, slices = 0, col_slice = 0, cols = 0, src = 0; // byte offsets in sweep_tab
-  } sweep[2];
-  // both directions' tables in one buffer, their values in one per precision
-  // (a few dozen buffers of their own took longer to set up than to fill)
-  DevBuf<char> sweep_tab;
+    int nb = 0;          // blocks of each direction
+    int gs[2] = {0, 0};
+    int max_loc[2] = {0, 0}, max_rows[2] = {0, 0}, max_slices[2] = {0, 0}, max_ent[2] = {0, 0};
+    int64_t updated[2] = {0, 0}; // updated rows over a direction's blocks
+    int64_t n_ent = 0;           // entries of both directions
+  } sweep;
+  DevBuf<SweepBlock> sweep_blocks; // both directions, nb each
+  DevBuf<int32_t> sweep_rows, sweep_col_slice, sweep_src;
+  DevBuf<SliceInfo> sweep_slices;
+  DevBuf<uint16_t> sweep_cols;
+  // the entries' values, then the second vector that the sweeps write while
+  // they read x, and the other way round; formed with the precision's first cycle
   DevBuf<double> sweep_v64;
   DevBuf<float> sweep_v32;
-  template <class U> const U *tab(int64_t off) const { return reinterpret_cast<const U *>(sweep_tab.p + off); }
-  DevBuf<double> y64;
-  DevBuf<float> y32;
   std::vector<int32_t> perm; // new -> old
   bool stream = false;       // matrix larger than the caches: non-temporal loads
   // value-only refresh of a lazy hierarchy: the level's CSR (levels >= 1),
@@ -1751,6 +1754,9 @@ struct afe_amg {
   CgScalars *h_sc = nullptr; // pinned
   double *h_rr = nullptr;    // pinned: the (r, r) partials of a CG iteration (RED_BLOCKS)
   bool has32 = false;
+  // the levels' sweep tables (as far as they have any), and their values per
+  // precision; short: there was no room for some
+  bool sweeps_formed = false, sweeps_ready[2] = {false, false}, sweeps_short = false;
   // captured V-cycles: [precision][symmetric]
   hipGraphExec_t vc_graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
   // captured CG iteration in two parts: [part][precision]; part 0 ends with
@@ -1827,7 +1833,6 @@ struct HostLevel {
   int cshift = 0;
   std::vector<int32_t> perm, iperm;
   std::vector<int32_t> smap, dsrc; // CSR entry -> layout position, row -> CSR diagonal
-  SweepTables sweep[2];            // blocks empty: one launch per colour
 };
 struct HostLayout {
   bool maps = false; // source maps for the value-only refresh
@@ -1887,47 +1892,14 @@ static void colour_code(HostLevel &hl) {
   hl.cshift = cshift;
 }
 
-// Levels whose sweeps run as one launch: of at most SWEEP_ROWS rows (larger
-// ones fill the chip with each colour and are bandwidth bound: with the bound at
-// 40K / 131K / 300K rows the CG of 263K P2 DOFs takes 9.02 / 9.03 / 9.66 ms,
-// the moving-mesh step of 251K P1 DOFs 6.78 / 6.65 / 6.86, the CG of 4.2M P2
-// DOFs 49.0 / 48.6 / 48.6 and 53.7 with its 481K-row level), of rows of at most
-// SWEEP_ROW_ENTRIES entries on average and with closures of at most
-// SWEEP_FACTOR times the level (the Galerkin levels of
-// tetrahedra couple 40 rows and more: a block's closure there is a large part
-// of the level).  Levels inside the dense sub-cycle need none, nor do the
-// server's hierarchies, which its batch runs with shared launches.
-// The tables cost set-up time: 16 hierarchies of 2K to 214K rows 504 -> 605 ms
-// (582 with 40K).  AFE_SWEEP_ROWS sets the bound for hierarchies built
-// afterwards (0: none).
-constexpr int64_t SWEEP_ROWS = 131072, SWEEP_ROW_ENTRIES = 24, SWEEP_BLOCK_MIN = 32, SWEEP_BLOCK_MAX = 320;
-constexpr double SWEEP_FACTOR = 6.0;
-static int64_t dense_rows_bound();
-
-static void build_sweeps(HostLevel &hl) {
-  const char *e = getenv("AFE_SWEEP_ROWS");
-  const int64_t most = e ? std::strtoll(e, nullptr, 10) : SWEEP_ROWS;
-  const int64_t n = hl.n;
-  if (t_first_fit_only || n > most || n <= dense_rows_bound() || hl.ncol < 2 || hl.ncol > 64 ||
-      (int64_t)hl.sa.cols.size() > SWEEP_ROW_ENTRIES * n)
-    return;
-  std::vector<int32_t> block_of;
-  // one block per CU
-  const int64_t target = std::min(SWEEP_BLOCK_MAX, std::max(SWEEP_BLOCK_MIN, (n + 255) / 256));
-  const int nb = sweep_partition(hl.sa, target, block_of);
-  if (!sweep_build(hl.sa, nb, block_of, false, SWEEP_FACTOR, hl.sweep[0]) ||
-      !sweep_build(hl.sa, nb, block_of, true, SWEEP_FACTOR, hl.sweep[1]))
-    hl.sweep[0] = hl.sweep[1] = SweepTables();
-}
-
 static void build_layout(const Hierarchy &h, HostLayout &lay, bool maps) {
   const int L = (int)h.A.size();
   lay.maps = maps && h.A[0].nnz() < INT32_MAX;
   lay.lv.assign(L, HostLevel());
   std::vector<std::vector<int32_t>> groups(L);
   // phase times for AFE_VERBOSE: colouring, row order, level sliced ELL,
-  // transfer operators, natural copy, sweep blocks
-  double tph[6] = {0, 0, 0, 0, 0, 0};
+  // transfer operators, natural copy
+  double tph[5] = {0, 0, 0, 0, 0};
   auto tick = [t = std::chrono::steady_clock::now()](double &acc) mutable {
     const auto now = std::chrono::steady_clock::now();
     acc += std::chrono::duration<double>(now - t).count();
@@ -1991,8 +1963,6 @@ static void build_layout(const Hierarchy &h, HostLayout &lay, bool maps) {
     if ((int64_t)hl.sa.cols.size() * 8 > stream_bytes() && hl.ncol <= CC_BASES && getenv("AFE_NO_C16") == nullptr)
       colour_code(hl);
     tick(tph[2]);
-    if (l + 1 < L) build_sweeps(hl);
-    tick(tph[5]);
     if (l + 1 < L) {
       build_sell(h.P[l], lay.lv[l + 1].perm, hl.iperm, {(int32_t)h.P[l].m}, false, hl.sp, nullptr, nullptr,
                  l == 0 ? 0 : lane_shift(h.P[l].m, 1, h.P[l].nnz()));
@@ -2055,10 +2025,8 @@ static void build_layout(const Hierarchy &h, HostLayout &lay, bool maps) {
     tick(tph[4]);
   }
   if (verbose())
-    fprintf(stderr,
-            "layout: colouring %.3f s, row order %.3f s, level ELL %.3f s, transfer %.3f s, natural %.3f s, "
-            "sweep blocks %.3f s\n",
-            tph[0], tph[1], tph[2], tph[3], tph[4], tph[5]);
+    fprintf(stderr, "layout: colouring %.3f s, row order %.3f s, level ELL %.3f s, transfer %.3f s, natural %.3f s\n",
+            tph[0], tph[1], tph[2], tph[3], tph[4]);
   if (h.full) {
     // the coarse vectors are in the level's colour order: permute the inverse
     const std::vector<int32_t> &pc = lay.lv[L - 1].perm;
@@ -2189,37 +2157,252 @@ static void ensure_dense(afe_amg *g, bool symmetric, int nu) {
   d.nu = nu;
 }
 
-// the blocks' value arrays and the second level vector
-static void alloc_sweeps(afe_amg *g, DevLevel &d) {
-  if (d.sweep[0].nb == 0) return;
-  const size_t n = (size_t)(d.sweep[0].n_ent + d.sweep[1].n_ent);
-  d.sweep_v64.alloc(g->ctx, n);
-  d.y64.alloc(g->ctx, d.n);
-  if (g->has32) {
-    d.sweep_v32.alloc(g->ctx, n);
-    d.y32.alloc(g->ctx, d.n);
+// Levels whose sweeps run as one launch: of at most SWEEP_ROWS rows (larger
+// ones fill the chip with each colour and are bandwidth bound: with the bound at
+// 40K / 131K / 300K rows the CG of 263K P2 DOFs takes 9.02 / 9.03 / 9.66 ms,
+// the moving-mesh step of 251K P1 DOFs 6.78 / 6.65 / 6.86, the CG of 4.2M P2
+// DOFs 49.0 / 48.6 / 48.6 and 53.7 with its 481K-row level), of at most
+// SWEEP_ROW_ENTRIES off-diagonal entries a row on average and with closures of
+// at most SWEEP_FACTOR times the level (the Galerkin levels of tetrahedra
+// couple 40 rows and more: a block's closure there is a large part of the
+// level).  Levels inside the dense sub-cycle need none.
+// AFE_SWEEP_ROWS sets the bound for hierarchies built afterwards (0: none);
+// the bit sets of the table kernels have to fit in LDS, which ends it near
+// 300K rows.
+constexpr int64_t SWEEP_ROWS = 131072, SWEEP_ROW_ENTRIES = 24, SWEEP_BLOCK_MIN = 32, SWEEP_BLOCK_MAX = 320;
+constexpr double SWEEP_FACTOR = 6.0;
+
+static int64_t sweep_set_lds(int64_t n) { return (n + 31) / 32 * 16; }
+
+static void choose_sweeps(afe_amg *g) {
+  const char *e = getenv("AFE_SWEEP_ROWS");
+  const int64_t most = e ? std::strtoll(e, nullptr, 10) : SWEEP_ROWS, dense = dense_rows_bound();
+  const int L = (int)g->lv.size();
+  for (int l = 0; l < L; l++) {
+    DevLevel &d = g->lv[l];
+    d.sweep_may = l + 1 < L && d.n <= most && d.n > dense && d.ncol >= 2 && d.ncol <= SWEEP_COLOURS &&
+                  g->h.A[l].nnz() - d.n <= SWEEP_ROW_ENTRIES * d.n && sweep_set_lds(d.n) + SWEEP_TABLE_LDS <= g->ctx->lds_bytes;
   }
 }
 
-// the blocks' values from the level's current ones
-static void fill_sweeps(afe_amg *g, DevLevel &d) {
-  for (DevLevel::Sweep &w : d.sweep)
-    if (w.nb > 0)
-      k_sweep_values<<<nblk(w.n_ent), 256, 0, g->ctx->stream>>>(
-          w.n_ent, d.tab<int32_t>(w.src), d.v64.p, d.sweep_v64.p + w.val0, d.v32.p,
-          g->has32 ? d.sweep_v32.p + w.val0 : nullptr);
+template <class T> static SweepLds sweep_lds_of(const DevLevel &d, int k) {
+  return sweep_lds<T>(d.sweep.max_loc[k], d.sweep.max_rows[k], d.sweep.max_slices[k], d.ncol, d.sweep.max_ent[k]);
+}
+template <class T> static bool sweeps_fit(const afe_amg *g, const DevLevel &d) {
+  return sweep_lds_of<T>(d, 0).total <= g->ctx->lds_bytes && sweep_lds_of<T>(d, 1).total <= g->ctx->lds_bytes;
+}
+
+static void drop_sweep(DevLevel &d) {
+  d.sweep = DevLevel::Sweep();
+  d.sweep_blocks.release();
+  d.sweep_rows.release();
+  d.sweep_col_slice.release();
+  d.sweep_src.release();
+  d.sweep_slices.release();
+  d.sweep_cols.release();
+  d.sweep_v64.release();
+  d.sweep_v32.release();
+}
+
+// The sweep tables of every level that may have them: the partition on the
+// host along the level's matrix, everything else on the device
+// (k_sweep_closure, k_sweep_rows, k_sweep_entries), each step for all levels
+// before the host waits for it.  Called before a hierarchy's first own cycle,
+// so that hierarchies which only join a batch never pay for it.
+// Creating a hierarchy takes what it takes without tables, 94 ms on 263K P2
+// DOFs, 125 on 251K P1 and 41 on 58K P2 (113, 145 and 56 with tables built on
+// the host for each); the first solve takes 2.3, 3.6 and 2.6 ms longer than
+// the second, about half of it the partition.
+static void form_sweeps(afe_amg *g) {
+  afe_ctx *ctx = g->ctx;
+  hipStream_t st = ctx->stream;
+  struct Work {
+    DevLevel *d;
+    int nb, W, steps;
+    std::vector<int32_t> head; // block of each stored row, then the colours' first rows
+    std::vector<int32_t> counts;
+    std::vector<SweepBlock> blocks;
+    int32_t *d_head, *d_counts;
+    uint32_t *d_bits;
+    SweepLevel lev;
+    int64_t rows = 0, slices = 0;
+  };
+  std::vector<Work> work;
+  size_t words = 0; // 32-bit words of workspace
+  for (size_t l = 0; l < g->lv.size(); l++) {
+    DevLevel &d = g->lv[l];
+    if (!d.sweep_may) continue;
+    work.emplace_back();
+    Work &w = work.back();
+    w.d = &d;
+    const int64_t n = d.n;
+    std::vector<int32_t> block_of;
+    // one block per CU
+    w.nb = sweep_partition(g->h.A[l], std::min(SWEEP_BLOCK_MAX, std::max(SWEEP_BLOCK_MIN, (n + 255) / 256)), d.perm,
+                           block_of);
+    w.W = (int)((n + 31) / 32);
+    w.head.resize(n + d.ncol + 1);
+    for (int64_t i = 0; i < n; i++) w.head[i] = block_of[d.perm[i]];
+    for (int c = 0; c <= d.ncol; c++) w.head[n + c] = d.colour_row[c];
+    w.counts.resize((size_t)2 * w.nb * (d.ncol + 2));
+    w.blocks.resize(2 * w.nb);
+    words += w.head.size() + w.counts.size() + (size_t)2 * w.nb * 2 * w.W;
+  }
+  if (work.empty()) return;
+  DevBuf<double> own;
+  int32_t *at = reinterpret_cast<int32_t *>(call_scratch(ctx, (words + 1) / 2, own));
+  for (Work &w : work) {
+    w.d_head = at;
+    at += w.head.size();
+    w.d_counts = at;
+    at += w.counts.size();
+    w.d_bits = reinterpret_cast<uint32_t *>(at);
+    at += (size_t)2 * w.nb * 2 * w.W;
+    HIPCHK(hipMemcpyAsync(w.d_head, w.head.data(), w.head.size() * 4, hipMemcpyHostToDevice, st));
+    w.lev = {(int)w.d->n, w.d->ncol, w.d->gs, w.d_head + w.d->n, w.d->col_slice.p, w.d->si.p, w.d->cols.p};
+  }
+  // (a kernel right behind queued host copies stalls the call)
+  HIPCHK(hipStreamSynchronize(st));
+  for (Work &w : work) {
+    k_sweep_closure<<<2 * w.nb, SWEEP_THREADS, (size_t)w.W * 8, st>>>(w.lev, w.d_head, w.nb, w.d_bits, w.d_counts);
+    HIPCHK(hipMemcpyAsync(w.counts.data(), w.d_counts, w.counts.size() * 4, hipMemcpyDeviceToHost, st));
+  }
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(st));
+  for (Work &w : work) {
+    DevLevel &d = *w.d;
+    DevLevel::Sweep s;
+    bool fits = true;
+    for (int k = 0; k < 2; k++) {
+      int64_t entries = 0;
+      auto count = [&](int b, int c) { return w.counts[(size_t)(k * w.nb + b) * (d.ncol + 2) + c]; };
+      for (int b = 0; b < w.nb; b++) {
+        for (int c = 0; c < d.ncol; c++) s.updated[k] += count(b, c);
+        entries += count(b, d.ncol + 1);
+      }
+      fits = fits && (double)s.updated[k] <= SWEEP_FACTOR * (double)d.n;
+      // lanes per row: a step's rows over the workgroup's lanes, at least an entry each
+      int &gs = s.gs[k];
+      while (gs < MAX_ROW_LANE_SHIFT && (int64_t(2) << gs) * s.updated[k] <= entries &&
+             (s.updated[k] << (gs + 1)) <= (int64_t)SWEEP_THREADS * w.nb * d.ncol)
+        gs++;
+      const int R = SELL_C >> gs;
+      for (int b = 0; b < w.nb; b++) {
+        SweepBlock &B = w.blocks[k * w.nb + b];
+        B = {(int32_t)std::min<int64_t>(w.rows, INT32_MAX), 0, 0, (int32_t)std::min<int64_t>(w.slices, INT32_MAX), 0, 0, 0};
+        for (int c = 0; c < d.ncol; c++) {
+          B.n_rows += count(b, c);
+          B.n_slices += (count(b, c) + R - 1) / R;
+        }
+        B.n_loc = B.n_rows + count(b, d.ncol);
+        w.rows += B.n_loc;
+        w.slices += B.n_slices;
+        s.max_loc[k] = std::max(s.max_loc[k], B.n_loc);
+        s.max_rows[k] = std::max(s.max_rows[k], B.n_rows);
+        s.max_slices[k] = std::max(s.max_slices[k], B.n_slices);
+      }
+      // local columns are 16 bits wide
+      fits = fits && s.max_loc[k] <= 65535 && w.rows <= INT32_MAX &&
+             sweep_set_lds(d.n) + 4 * s.max_slices[k] + SWEEP_TABLE_LDS <= ctx->lds_bytes;
+    }
+    if (!fits) continue; // d.sweep stays without blocks
+    s.nb = w.nb;
+    d.sweep = s;
+    d.sweep_rows.alloc(ctx, w.rows);
+    d.sweep_slices.alloc(ctx, w.slices);
+    d.sweep_col_slice.alloc(ctx, (size_t)2 * w.nb * (d.ncol + 1));
+    d.sweep_blocks.upload(ctx, w.blocks);
+  }
+  HIPCHK(hipStreamSynchronize(st));
+  for (Work &w : work) {
+    DevLevel &d = *w.d;
+    if (d.sweep.nb == 0) continue;
+    const int most = std::max(d.sweep.max_slices[0], d.sweep.max_slices[1]);
+    k_sweep_rows<<<2 * w.nb, SWEEP_THREADS, (size_t)sweep_set_lds(d.n) + 4 * most, st>>>(
+        w.lev, w.d_head, w.nb, w.d_bits, w.d_counts, d.sweep.gs[0], d.sweep.gs[1], d.sweep_blocks.p, d.sweep_rows.p,
+        d.sweep_slices.p, d.sweep_col_slice.p);
+    HIPCHK(hipMemcpyAsync(w.blocks.data(), d.sweep_blocks.p, w.blocks.size() * sizeof(SweepBlock),
+                          hipMemcpyDeviceToHost, st));
+  }
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(st));
+  for (Work &w : work) {
+    DevLevel &d = *w.d;
+    if (d.sweep.nb == 0) continue;
+    for (int b = 0; b < 2 * w.nb; b++) {
+      SweepBlock &B = w.blocks[b];
+      B.ent0 = (int32_t)std::min<int64_t>(d.sweep.n_ent, INT32_MAX);
+      d.sweep.n_ent += B.n_ent;
+      d.sweep.max_ent[b / w.nb] = std::max(d.sweep.max_ent[b / w.nb], B.n_ent);
+    }
+    if (d.sweep.n_ent > INT32_MAX || (!sweeps_fit<float>(g, d) && !sweeps_fit<double>(g, d))) {
+      drop_sweep(d);
+      continue;
+    }
+    d.sweep_cols.alloc(ctx, d.sweep.n_ent);
+    d.sweep_src.alloc(ctx, d.sweep.n_ent);
+    d.sweep_blocks.upload(ctx, w.blocks);
+  }
+  HIPCHK(hipStreamSynchronize(st));
+  for (Work &w : work) {
+    DevLevel &d = *w.d;
+    if (d.sweep.nb == 0) continue;
+    k_sweep_entries<<<2 * w.nb, SWEEP_THREADS, (size_t)sweep_set_lds(d.n), st>>>(
+        w.lev, w.nb, w.d_bits, d.sweep.gs[0], d.sweep.gs[1], d.sweep_blocks.p, d.sweep_rows.p, d.sweep_slices.p,
+        d.sweep_col_slice.p, d.sweep_cols.p, d.sweep_src.p);
+  }
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(st)); // the workspace is free again
+}
+
+template <class T> static DevBuf<T> &sweep_buf(DevLevel &d);
+template <> DevBuf<double> &sweep_buf<double>(DevLevel &d) { return d.sweep_v64; }
+template <> DevBuf<float> &sweep_buf<float>(DevLevel &d) { return d.sweep_v32; }
+
+// the blocks' values of precision T, where there are any, from the level's current ones
+template <class T> static void fill_sweeps(afe_amg *g, DevLevel &d) {
+  if (!sweep_buf<T>(d).p) return;
+  const T *level;
+  if constexpr (std::is_same<T, double>::value) level = d.v64.p;
+  else level = d.v32.p;
+  k_sweep_values<T><<<nblk(d.sweep.n_ent), 256, 0, g->ctx->stream>>>(d.sweep.n_ent, d.sweep_src.p, level,
+                                                                     sweep_buf<T>(d).p);
   HIPCHK(hipGetLastError());
 }
 
-template <class T> static SweepLds sweep_lds_of(const DevLevel::Sweep &w) {
-  return sweep_lds<T>(w.max_loc, w.max_rows, w.max_slices, w.ncol, w.max_ent);
+// whether level d's sweeps run as one launch in precision T
+template <class T> static bool sweeps_fused(DevLevel &d) { return d.sweep.nb > 0 && sweep_buf<T>(d).p; }
+
+// before a cycle in precision T: the sweep tables, and the precision's values
+// of them.  Without room for them the levels keep one launch per colour, until
+// new values come.
+template <class T> static void ensure_sweeps(afe_amg *g, int nu) {
+  bool &ready = g->sweeps_ready[std::is_same<T, float>::value ? 1 : 0];
+  if (nu == 0 || ready) return;
+  try {
+    if (!g->sweeps_formed) form_sweeps(g);
+    g->sweeps_formed = true;
+    for (DevLevel &d : g->lv) {
+      if (d.sweep.nb == 0 || !sweeps_fit<T>(g, d)) continue;
+      sweep_buf<T>(d).alloc(g->ctx, d.sweep.n_ent + d.n);
+      fill_sweeps<T>(g, d);
+    }
+  } catch (const afe::Error &x) {
+    if (x.code != AFE_E_NOMEM) throw;
+    for (DevLevel &d : g->lv) {
+      sweep_buf<T>(d).release();
+      if (!g->sweeps_formed) drop_sweep(d);
+    }
+    g->sweeps_short = true;
+  }
+  ready = true;
 }
 
-// whether level d's sweeps run as one launch in precision T
-template <class T> static bool sweeps_fused(const afe_amg *g, const DevLevel &d) {
-  for (const DevLevel::Sweep &w : d.sweep)
-    if (w.nb == 0 || sweep_lds_of<T>(w).total > g->ctx->lds_bytes) return false;
-  return true;
+// after new values or a new layout: what had no room is tried again
+static void retry_sweeps(afe_amg *g) {
+  if (!g->sweeps_short) return;
+  g->sweeps_short = g->sweeps_ready[0] = g->sweeps_ready[1] = false;
+  drop_graphs(g);
 }
 
 static void finish_levels(afe_amg *g);
@@ -2275,41 +2458,6 @@ static void upload_layout(afe_amg *g, HostLayout &lay) {
         d.t_v32.upload(ctx, to_prec<float>(st.vals));
       }
     }
-    std::vector<char> tab;
-    int64_t val0 = 0;
-    for (int k = 0; k < 2; k++) {
-      const SweepTables &t = hl.sweep[k];
-      DevLevel::Sweep &w = d.sweep[k];
-      w.nb = (int)t.blocks.size();
-      if (w.nb == 0) continue;
-      w.ncol = t.ncol;
-      w.gs = t.gshift;
-      w.max_loc = t.max_loc;
-      w.max_rows = t.max_rows;
-      w.max_slices = t.max_slices;
-      w.max_ent = t.max_ent;
-      w.n_ent = (int64_t)t.src.size();
-      w.val0 = val0;
-      val0 += w.n_ent;
-      auto put = [&](const auto &v) {
-        const int64_t off = (int64_t)(tab.size() + 255) / 256 * 256;
-        const char *p = reinterpret_cast<const char *>(v.data());
-        tab.resize(off);
-        tab.insert(tab.end(), p, p + v.size() * sizeof(v[0]));
-        return off;
-      };
-      w.blocks = put(t.blocks);
-      w.rows = put(t.rows);
-      w.slices = put(t.slices);
-      w.col_slice = put(t.col_slice);
-      w.cols = put(t.cols);
-      w.src = put(t.src);
-    }
-    if (!tab.empty()) {
-      d.sweep_tab.upload(ctx, tab);
-      HIPCHK(hipStreamSynchronize(ctx->stream)); // tab goes out of scope
-    }
-    alloc_sweeps(g, d);
     d.x64.alloc(ctx, d.n);
     d.b64.alloc(ctx, d.n);
     d.t64.alloc(ctx, d.n);
@@ -2369,8 +2517,6 @@ static void upload_layout(afe_amg *g, HostLayout &lay) {
   while (g->tail0 > 0 && g->lv[g->tail0 - 1].n <= g_tune.tail_rows) g->tail0--;
   if (h.full) g->minv.upload(ctx, lay.minv_perm);
   finish_levels(g); // returns with the copies finished
-  for (DevLevel &d : g->lv) fill_sweeps(g, d);
-  HIPCHK(hipStreamSynchronize(ctx->stream));
 }
 
 // the level descriptors of the tail and batch kernels (device pointers into
@@ -2379,6 +2525,8 @@ static void finish_levels(afe_amg *g) {
   afe_ctx *ctx = g->ctx;
   const int L = (int)g->lv.size();
   choose_dense_level(g);
+  choose_sweeps(g);
+  g->sweeps_formed = g->sweeps_short = g->sweeps_ready[0] = g->sweeps_ready[1] = false;
   std::vector<LevelDev<double>> d64(L);
   std::vector<LevelDev<float>> d32(L);
   for (int l = 0; l < L; l++) {
@@ -2568,7 +2716,8 @@ static void device_lazy_refresh(afe_amg *g, afe_matrix *a) {
     k_refresh_vals<<<nblk(nnz), 256, 0, s>>>(nnz, lvals(l), d.smap.p, d.v64.p, g->has32 ? d.v32.p : nullptr);
     k_refresh_diag<<<nblk(d.n), 256, 0, s>>>(d.n, lvals(l), d.dsrc.p, d.diag64.p, d.invd64.p,
                                              g->has32 ? d.diag32.p : nullptr, g->has32 ? d.invd32.p : nullptr);
-    fill_sweeps(g, d);
+    fill_sweeps<double>(g, d);
+    fill_sweeps<float>(g, d);
   }
   const int64_t n0 = g->lv[0].n, nnz0 = h.A[0].nnz();
   k_refresh_vals<<<nblk(nnz0), 256, 0, s>>>(nnz0, a->val.p, g->nat_smap.p, g->nat_v64.p, nullptr);
@@ -2590,6 +2739,7 @@ static void device_lazy_refresh(afe_amg *g, afe_matrix *a) {
   g->A0 = a;
   g->host_vals_stale = true;
   drop_dense(g);
+  retry_sweeps(g);
 }
 
 // host copies of the level values after device refreshes
@@ -2765,9 +2915,6 @@ extern "C" int afe_amg_clone(const afe_amg *src, afe_matrix *a, afe_amg **out) {
     clone_buf(ctx, d.c_val, o.c_val);
     clone_buf(ctx, d.P_val, o.P_val);
     clone_buf(ctx, d.Pt_val, o.Pt_val);
-    for (int k = 0; k < 2; k++) d.sweep[k] = o.sweep[k];
-    clone_buf(ctx, d.sweep_tab, o.sweep_tab);
-    alloc_sweeps(g.get(), d); // the values come with the refresh below
     d.x64.alloc(ctx, d.n);
     d.b64.alloc(ctx, d.n);
     d.t64.alloc(ctx, d.n);
@@ -2857,8 +3004,6 @@ template <> struct Prec<double> {
   static double *x(DevLevel &d) { return d.x64.p; }
   static double *b(DevLevel &d) { return d.b64.p; }
   static double *t(DevLevel &d) { return d.t64.p; }
-  static double *y(DevLevel &d) { return d.y64.p; }
-  static const double *sv(const DevLevel &d) { return d.sweep_v64.p; }
   static const LevelDev<double> *ld(afe_amg *g) { return g->ld64.p; }
 };
 template <> struct Prec<float> {
@@ -2870,8 +3015,6 @@ template <> struct Prec<float> {
   static float *x(DevLevel &d) { return d.x32.p; }
   static float *b(DevLevel &d) { return d.b32.p; }
   static float *t(DevLevel &d) { return d.t32.p; }
-  static float *y(DevLevel &d) { return d.y32.p; }
-  static const float *sv(const DevLevel &d) { return d.sweep_v32.p; }
   static const LevelDev<float> *ld(afe_amg *g) { return g->ld32.p; }
 };
 
@@ -2903,23 +3046,23 @@ static void issue_vcycle(afe_amg *g, int nu, bool symmetric, hipStream_t st, boo
   int top = dense ? std::min(g->tail0, g->dense_level) : g->tail0;
   if (dense && nu > 0) {
     int t = top;
-    while (t < g->dense_level && sweeps_fused<T>(g, g->lv[t])) t++;
+    while (t < g->dense_level && sweeps_fused<T>(g->lv[t])) t++;
     if (t == g->dense_level) top = t;
   }
   const bool to_tail = top < (dense ? g->dense_level : Lc);
   // one-launch sweeps alternate between the level's x and y: at[l] is the one
   // that holds the current iterate (x again after the 2 nu sweeps)
   std::vector<int> at(top, 0);
-  auto fused = [&](DevLevel &d) { return nu > 0 && sweeps_fused<T>(g, d); };
-  auto vec = [&](DevLevel &d, int k) { return k ? Prec<T>::y(d) : Prec<T>::x(d); };
+  auto fused = [&](DevLevel &d) { return nu > 0 && sweeps_fused<T>(d); };
+  auto vec = [&](DevLevel &d, int k) { return k ? sweep_buf<T>(d).p + d.sweep.n_ent : Prec<T>::x(d); };
   auto sweep = [&](DevLevel &d, int &k, bool rev, bool zero, DevLevel *dn) {
-    const DevLevel::Sweep &w = d.sweep[rev ? 1 : 0];
-    const SweepLds lds = sweep_lds_of<T>(w);
-    k_sweep<T><<<w.nb, SWEEP_THREADS, (size_t)lds.total, st>>>(
-        d.tab<SweepBlock>(w.blocks), d.tab<int32_t>(w.rows), d.tab<SliceInfo>(w.slices),
-        d.tab<int32_t>(w.col_slice), d.tab<uint16_t>(w.cols), Prec<T>::sv(d) + w.val0, w.ncol, w.gs, lds,
+    const int r = rev ? 1 : 0, nb = d.sweep.nb;
+    const SweepLds lds = sweep_lds_of<T>(d, r);
+    k_sweep<T><<<nb, SWEEP_THREADS, (size_t)lds.total, st>>>(
+        d.sweep_blocks.p + r * nb, d.sweep_rows.p, d.sweep_slices.p, d.sweep_col_slice.p + r * nb * (d.ncol + 1),
+        d.sweep_cols.p, sweep_buf<T>(d).p, d.ncol, d.sweep.gs[r], lds,
         Prec<T>::invd(d), Prec<T>::b(d), zero ? nullptr : vec(d, k), d.t_si.p, d.t_cols.p, Prec<T>::tv(d),
-        dn ? Prec<T>::x(*dn) : nullptr, vec(d, 1 - k), rev ? 1 : 0);
+        dn ? Prec<T>::x(*dn) : nullptr, vec(d, 1 - k), r);
     k = 1 - k;
   };
   for (int l = 0; l < top; l++) {
@@ -3032,6 +3175,8 @@ static bool use_graphs() {
 static void launch_graph_or_issue(afe_amg *g, int prec, bool symmetric, int nu) {
   hipStream_t st = g->ctx->stream;
   ensure_dense(g, symmetric, nu);
+  if (prec == 1) ensure_sweeps<float>(g, nu);
+  else ensure_sweeps<double>(g, nu);
   if (!use_graphs()) {
     if (prec == 1)
       issue_vcycle<float>(g, nu, symmetric, st, symmetric);
@@ -3606,6 +3751,22 @@ extern "C" int afe_amg_device_info(const afe_amg *g, int32_t level, int64_t *row
   if (stored) *stored = (int64_t)d.cols.n;
   if (tail_level) *tail_level = g->tail0;
   if (row_lanes) *row_lanes = 1 << d.gs;
+  return AFE_OK;
+}
+
+// the block sweeps of a level: blocks per direction (0: one launch per colour,
+// or no own cycle yet), rows that the forward / reverse blocks update together,
+// and whether FP64 / FP32 sweeps run as one launch
+extern "C" int afe_amg_sweep_info(const afe_amg *g, int32_t level, int32_t *blocks, int64_t *updated, int32_t *fused) {
+  if (!g || !g->ctx || level < 0 || level >= (int)g->lv.size()) return fail(AFE_E_ARG, "bad level");
+  const DevLevel &d = g->lv[level];
+  if (blocks) *blocks = d.sweep.nb;
+  if (updated)
+    for (int k = 0; k < 2; k++) updated[k] = d.sweep.updated[k];
+  if (fused) {
+    fused[0] = d.sweep.nb > 0 && d.sweep_v64.p;
+    fused[1] = d.sweep.nb > 0 && d.sweep_v32.p;
+  }
   return AFE_OK;
 }
 

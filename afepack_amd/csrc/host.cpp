@@ -10,7 +10,6 @@
 #include <omp.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -967,33 +966,20 @@ void build_sell(const Csr &a, const std::vector<int32_t> &perm,
 // ===========================================================================
 // colour sweeps by independent blocks
 // ===========================================================================
-// f(column, position) for the stored entries of a row (padding left out)
-template <class F> static inline void sell_row(const Sell &sa, int32_t row, const std::vector<int32_t> &slice_of, F f) {
-  const SliceInfo &si = sa.slices[slice_of[row]];
-  const int G = 1 << sa.gshift, l = row - si.row0;
-  for (int32_t s = 0; s < si.width; s++)
-    for (int k = 0; k < G; k++) {
-      const int32_t pos = si.off + s * SELL_C + (l << sa.gshift) + k;
-      if (sa.cols[pos] != row) f(sa.cols[pos], pos);
-    }
+// f(column) for the off-diagonal entries of a row
+template <class F> static inline void off_diagonals(const Csr &a, int32_t i, F f) {
+  for (int64_t k = a.rp[i]; k < a.rp[i + 1]; k++)
+    if (a.col[k] != i) f(a.col[k]);
 }
 
-static std::vector<int32_t> sell_slice_of(const Sell &sa) {
-  std::vector<int32_t> so(sa.n_rows);
-  for (size_t s = 0; s < sa.slices.size(); s++)
-    for (int32_t l = 0; l < sa.slices[s].nrow; l++) so[sa.slices[s].row0 + l] = (int32_t)s;
-  return so;
-}
-
-int sweep_partition(const Sell &sa, int64_t target, std::vector<int32_t> &block_of) {
-  const int64_t n = sa.n_rows;
-  const std::vector<int32_t> so = sell_slice_of(sa);
+int sweep_partition(const Csr &a, int64_t target, const std::vector<int32_t> &order, std::vector<int32_t> &block_of) {
+  const int64_t n = a.m;
   block_of.assign(n, -1);
   std::vector<int32_t> queue;
   queue.reserve(target * 8);
   int nb = 0;
   // seeds: where the last block's growth stopped (so that blocks tile), else
-  // the first row left
+  // the first row left in the given order
   std::vector<int32_t> front;
   size_t front_at = 0;
   int64_t scan = 0;
@@ -1004,7 +990,7 @@ int sweep_partition(const Sell &sa, int64_t target, std::vector<int32_t> &block_
       front_at++;
     }
     while (seed < 0 && scan < n) {
-      if (block_of[scan] < 0) seed = (int32_t)scan;
+      if (block_of[order[scan]] < 0) seed = order[scan];
       scan++;
     }
     if (seed < 0) break;
@@ -1013,7 +999,7 @@ int sweep_partition(const Sell &sa, int64_t target, std::vector<int32_t> &block_
     block_of[seed] = nb;
     int64_t size = 1;
     for (size_t h = 0; h < queue.size(); h++)
-      sell_row(sa, queue[h], so, [&](int32_t c, int32_t) {
+      off_diagonals(a, queue[h], [&](int32_t c) {
         if (block_of[c] >= 0) return;
         if (size < target) {
           block_of[c] = nb;
@@ -1030,8 +1016,8 @@ int sweep_partition(const Sell &sa, int64_t target, std::vector<int32_t> &block_
   std::vector<int64_t> size(nb, 0);
   for (int64_t i = 0; i < n; i++) size[block_of[i]]++;
   std::vector<std::vector<int32_t>> small(nb);
-  for (int64_t i = 0; i < n; i++)
-    if (size[block_of[i]] * 4 < target) small[block_of[i]].push_back((int32_t)i);
+  for (int32_t i : order)
+    if (size[block_of[i]] * 4 < target) small[block_of[i]].push_back(i);
   std::vector<int32_t> votes(nb, 0), seen;
   std::vector<int32_t> into(nb);
   std::iota(into.begin(), into.end(), 0);
@@ -1039,7 +1025,7 @@ int sweep_partition(const Sell &sa, int64_t target, std::vector<int32_t> &block_
     if (small[b].empty()) continue;
     seen.clear();
     for (int32_t i : small[b])
-      sell_row(sa, i, so, [&](int32_t c, int32_t) {
+      off_diagonals(a, i, [&](int32_t c) {
         const int32_t o = block_of[c];
         if (o == b || !small[o].empty()) return;
         if (votes[o]++ == 0) seen.push_back(o);
@@ -1056,152 +1042,6 @@ int sweep_partition(const Sell &sa, int64_t target, std::vector<int32_t> &block_
     if (into[b] == b) number[b] = count++;
   for (int64_t i = 0; i < n; i++) block_of[i] = number[into[block_of[i]]];
   return count;
-}
-
-bool sweep_build(const Sell &sa, int n_blocks, const std::vector<int32_t> &block_of, bool reverse,
-                 double max_factor, SweepTables &out) {
-  const int64_t n = sa.n_rows;
-  const int ncol = (int)sa.group_row.size() - 1;
-  const std::vector<int32_t> so = sell_slice_of(sa);
-  std::vector<int32_t> colour(n);
-  for (int c = 0; c < ncol; c++)
-    for (int32_t r = sa.group_row[c]; r < sa.group_row[c + 1]; r++) colour[r] = c;
-  std::vector<int64_t> bptr(n_blocks + 1, 0);
-  std::vector<int32_t> brows(n);
-  for (int64_t i = 0; i < n; i++) bptr[block_of[i] + 1]++;
-  for (int b = 0; b < n_blocks; b++) bptr[b + 1] += bptr[b];
-  {
-    std::vector<int64_t> fill(bptr.begin(), bptr.end() - 1);
-    for (int64_t i = 0; i < n; i++) brows[fill[block_of[i]]++] = (int32_t)i;
-  }
-  struct Part {
-    int32_t n_rows = 0;
-    std::vector<int32_t> rows, src;
-    std::vector<uint16_t> cols;
-    std::vector<int32_t> count; // updated rows per colour
-  };
-  std::vector<Part> parts(n_blocks);
-  int64_t updated = 0, entries = 0;
-  std::atomic<int64_t> total{0};
-  const double limit = max_factor * (double)n;
-  // the closures
-#pragma omp parallel reduction(+ : updated, entries)
-  {
-    std::vector<int32_t> stamp(n, -1), list;
-#pragma omp for schedule(dynamic, 4)
-    for (int b = 0; b < n_blocks; b++) {
-      if ((double)total.load(std::memory_order_relaxed) > limit) continue; // too many already
-      list.assign(brows.begin() + bptr[b], brows.begin() + bptr[b + 1]);
-      for (int32_t i : list) stamp[i] = b;
-      for (size_t h = 0; h < list.size(); h++) {
-        const int32_t i = list[h], ci = colour[i];
-        sell_row(sa, i, so, [&](int32_t j, int32_t) {
-          const bool earlier = reverse ? colour[j] > ci : colour[j] < ci;
-          if (earlier && stamp[j] != b) {
-            stamp[j] = b;
-            list.push_back(j);
-          }
-          entries++;
-        });
-      }
-      Part &p = parts[b];
-      p.count.assign(ncol, 0);
-      std::sort(list.begin(), list.end()); // stored order: by colour
-      for (int32_t i : list) p.count[colour[i]]++;
-      p.n_rows = (int32_t)list.size();
-      p.rows = list;
-      updated += p.n_rows;
-      total += p.n_rows;
-    }
-  }
-  if ((double)updated > limit) return false;
-  // lanes per row: a step's rows over the workgroup's lanes, at least an entry each
-  int gs = 0;
-  const int64_t steps = (int64_t)n_blocks * ncol;
-  while (gs < MAX_ROW_LANE_SHIFT && (int64_t(2) << gs) * updated <= entries && (updated << (gs + 1)) <= SWEEP_THREADS * steps) gs++;
-  const int G = 1 << gs, R = SELL_C >> gs;
-  std::vector<std::vector<SliceInfo>> slices(n_blocks);
-  std::vector<int32_t> col_slice((size_t)n_blocks * (ncol + 1));
-#pragma omp parallel
-  {
-    std::vector<int32_t> local(n, -1);
-#pragma omp for schedule(dynamic, 4)
-    for (int b = 0; b < n_blocks; b++) {
-      Part &p = parts[b];
-      for (int32_t l = 0; l < p.n_rows; l++) local[p.rows[l]] = l;
-      int32_t r = 0, off = 0;
-      std::vector<std::pair<int32_t, int32_t>> ent;
-      for (int c = 0; c <= ncol; c++) {
-        col_slice[(size_t)b * (ncol + 1) + c] = (int32_t)slices[b].size();
-        if (c == ncol) break;
-        const int32_t rend = r + p.count[c];
-        for (int32_t r0 = r; r0 < rend; r0 += R) {
-          const int32_t nrow = std::min(R, rend - r0);
-          int32_t width = 0;
-          for (int32_t l = 0; l < nrow; l++) {
-            int32_t len = 0;
-            sell_row(sa, p.rows[r0 + l], so, [&](int32_t, int32_t) { len++; });
-            width = std::max(width, (len + G - 1) >> gs);
-          }
-          slices[b].push_back({r0, nrow, width, off});
-          p.cols.resize(off + width * SELL_C, 0);
-          p.src.resize(off + width * SELL_C, -1);
-          for (int32_t l = 0; l < nrow; l++) {
-            int32_t j = 0;
-            sell_row(sa, p.rows[r0 + l], so, [&](int32_t col, int32_t pos) {
-              if (local[col] < 0) {
-                local[col] = (int32_t)p.rows.size();
-                p.rows.push_back(col);
-              }
-              const int32_t q = off + (j >> gs) * SELL_C + (l << gs) + (j & (G - 1));
-              p.cols[q] = (uint16_t)local[col];
-              p.src[q] = pos;
-              j++;
-            });
-            for (; j < width << gs; j++)
-              p.cols[off + (j >> gs) * SELL_C + (l << gs) + (j & (G - 1))] = (uint16_t)(r0 + l);
-          }
-          off += width * SELL_C;
-        }
-        r = rend;
-      }
-      for (int32_t i : p.rows) local[i] = -1;
-    }
-  }
-  out = SweepTables();
-  out.ncol = ncol;
-  out.gshift = gs;
-  out.updated = updated;
-  out.blocks.resize(n_blocks);
-  int64_t row0 = 0, slice0 = 0, ent0 = 0;
-  for (int b = 0; b < n_blocks; b++) {
-    const Part &p = parts[b];
-    out.blocks[b] = {(int32_t)row0, p.n_rows, (int32_t)p.rows.size(), (int32_t)slice0, (int32_t)slices[b].size(),
-                     (int32_t)ent0, (int32_t)p.cols.size()};
-    out.max_loc = std::max(out.max_loc, (int)p.rows.size());
-    out.max_rows = std::max(out.max_rows, (int)p.n_rows);
-    out.max_slices = std::max(out.max_slices, (int)slices[b].size());
-    out.max_ent = std::max(out.max_ent, (int)p.cols.size());
-    row0 += (int64_t)p.rows.size();
-    slice0 += (int64_t)slices[b].size();
-    ent0 += (int64_t)p.cols.size();
-  }
-  if (ent0 > INT32_MAX || row0 > INT32_MAX || out.max_loc > 65535) return false;
-  out.rows.resize(row0);
-  out.slices.resize(slice0);
-  out.cols.resize(ent0);
-  out.src.resize(ent0);
-  out.col_slice = std::move(col_slice);
-#pragma omp parallel for schedule(static)
-  for (int b = 0; b < n_blocks; b++) {
-    const SweepBlock &k = out.blocks[b];
-    const Part &p = parts[b];
-    for (int32_t l = 0; l < k.n_loc; l++) out.rows[k.row0 + l] = block_of[p.rows[l]] == b ? ~p.rows[l] : p.rows[l];
-    std::copy(slices[b].begin(), slices[b].end(), out.slices.begin() + k.slice0);
-    std::copy(p.cols.begin(), p.cols.end(), out.cols.begin() + k.ent0);
-    std::copy(p.src.begin(), p.src.end(), out.src.begin() + k.ent0);
-  }
-  return true;
 }
 
 // host threads of the parallel loops started by the calling thread

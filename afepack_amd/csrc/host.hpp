@@ -169,33 +169,19 @@ int row_lane_shift(int64_t rows, int64_t groups, int64_t entries, int max_shift)
 // closure's other neighbours enter with the values from before the sweep, so
 // a block needs nothing from the others, and every block computes a row that
 // several of them update from the same operands.
-// Tables of all blocks, one after another.  A block's local rows are its
-// closure, by colour, then the neighbours it only reads (halo).
+// A block's local rows are its closure, by colour, then the neighbours it only
+// reads (halo).  The blocks of the forward sweep come first, then those of the
+// reverse one; their tables lie one after another.
 constexpr int SWEEP_THREADS = 1024; // of the workgroup that runs a block
 struct SweepBlock {
   int32_t row0, n_rows, n_loc; // rows[row0 ..): n_rows updated rows, n_loc local rows in all
   int32_t slice0, n_slices;    // slices[slice0 ..): row0 / off of a slice are local to the block
   int32_t ent0, n_ent;         // cols / src [ent0 ..)
 };
-struct SweepTables {
-  int ncol = 0, gshift = 0;
-  int max_loc = 0, max_rows = 0, max_slices = 0, max_ent = 0; // largest block
-  int64_t updated = 0;              // updated rows over all blocks
-  std::vector<SweepBlock> blocks;
-  std::vector<int32_t> rows;        // local row -> stored row of the level; own rows as ~row
-  std::vector<SliceInfo> slices;
-  std::vector<int32_t> col_slice;   // per block: ncol + 1 slice bounds
-  std::vector<uint16_t> cols;       // local columns (padding: a local row)
-  std::vector<int32_t> src;         // position in the level's layout, -1 for padding
-};
 // block_of: row -> block, for blocks of about `target` rows grown breadth
-// first along the layout's entries
-int sweep_partition(const Sell &sa, int64_t target, std::vector<int32_t> &block_of);
-// tables of one sweep direction (reverse: colours from the last to the
-// first); false when the updated rows exceed max_factor times the level's, or
-// a block's local rows 2^16
-bool sweep_build(const Sell &sa, int n_blocks, const std::vector<int32_t> &block_of, bool reverse,
-                 double max_factor, SweepTables &out);
+// first along the matrix's off-diagonal entries, the first from order[0];
+// returns the number of blocks
+int sweep_partition(const Csr &a, int64_t target, const std::vector<int32_t> &order, std::vector<int32_t> &block_of);
 
 // colouring of the symmetrised graph of the stored off-diagonal entries
 // (explicit zeros included): DSatur for matrices of at most dsatur_max_rows

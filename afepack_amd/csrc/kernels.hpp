@@ -1235,7 +1235,7 @@ __global__ __launch_bounds__(BLK) void k_prolong(const SliceInfo *__restrict__ s
 }
 
 // ---------------------------------------------------------------------------
-// a whole colour sweep of a small level in one launch (SweepTables): block k
+// a whole colour sweep of a small level in one launch: block k
 // loads x of its local rows (zero without xin; with xc, x + P^T xc, the
 // prolongation), runs the colours on its closure in LDS and writes its own
 // rows to xout, another buffer than xin, from which other blocks still read.
@@ -1411,15 +1411,252 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep(
   }
 }
 
+// ---------------------------------------------------------------------------
+// the tables of k_sweep from a level's layout and a partition of its rows,
+// formed on the device: workgroup k takes block k of the forward sweep or, from
+// nb on, block k - nb of the reverse one.  The rows of the closure and of the
+// halo are bit sets in LDS; the stored order is by colour, so "of an earlier
+// colour" is a comparison with the row's colour bounds, a local row's number is
+// its rank in the set, and one pass over the colours, from the one swept last
+// to the one swept first, closes the set.  Latency bound: 512 workgroups of
+// dependent loads over rows that share caches.
+// ---------------------------------------------------------------------------
+struct SweepLevel { // a level's sliced-ELL layout, as the table kernels read it
+  int n, ncol, gs;
+  const int32_t *colour_row, *colour_slice; // first row / slice of each colour
+  const SliceInfo *si;
+  const int32_t *cols;
+};
+constexpr int SWEEP_COLOURS = 64; // k_sweep holds a step per lane
+constexpr int SWEEP_TABLE_LDS = 4096; // the table kernels' static LDS beyond what all kernels leave
+
+// f(column, position) for the entries of stored row r of colour c, in stored
+// order (padding names the row itself)
+template <class F> __device__ __forceinline__ void sweep_row(const SweepLevel &L, int r, int c, int c_row0, F f) {
+  const int i = r - c_row0, R = WAVE >> L.gs, G = 1 << L.gs;
+  const SliceInfo q = L.si[L.colour_slice[c] + i / R];
+  const int at = q.off + ((i % R) << L.gs);
+  for (int j = 0; j < q.width << L.gs; j++) {
+    const int pos = at + (j >> L.gs) * WAVE + (j & (G - 1));
+    const int col = L.cols[pos];
+    if (col != r) f(col, pos);
+  }
+}
+
+// put(i, sum of f before i) for i < m; returns the sum (in every thread)
+template <class F, class P> __device__ __forceinline__ int sweep_scan(int m, int *part, F f, P put) {
+  const int tid = threadIdx.x, per = (m + SWEEP_THREADS - 1) / SWEEP_THREADS;
+  const int i0 = tid * per < m ? tid * per : m, i1 = i0 + per < m ? i0 + per : m;
+  int s = 0;
+  for (int i = i0; i < i1; i++) s += f(i);
+  part[tid] = s;
+  __syncthreads();
+  for (int d = 1; d < SWEEP_THREADS; d <<= 1) {
+    const int v = tid >= d ? part[tid - d] : 0;
+    __syncthreads();
+    part[tid] += v;
+    __syncthreads();
+  }
+  int run = part[tid] - s;
+  for (int i = i0; i < i1; i++) {
+    const int v = f(i);
+    put(i, run);
+    run += v;
+  }
+  const int total = part[SWEEP_THREADS - 1];
+  __syncthreads();
+  return total;
+}
+
+__device__ __forceinline__ bool sweep_bit(const uint32_t *set, int r) { return set[r >> 5] >> (r & 31) & 1u; }
+__device__ __forceinline__ int sweep_rank(const uint32_t *set, const int *before, int r) {
+  return before[r >> 5] + __popc(set[r >> 5] & ((1u << (r & 31)) - 1u));
+}
+
+// bits: per workgroup the closure's set, then the halo's, (n + 31) / 32 words
+// each; counts: per workgroup the closure's rows of each colour, the halo's
+// rows, the closure's entries
+__global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_closure(SweepLevel L, const int32_t *__restrict__ block_of,
+                                                                 int nb, uint32_t *__restrict__ bits,
+                                                                 int32_t *__restrict__ counts) {
+  extern __shared__ __align__(16) char sweep_smem[];
+  __shared__ int s_row[SWEEP_COLOURS + 1], s_cnt[SWEEP_COLOURS + 2];
+  const int W = (L.n + 31) / 32, tid = threadIdx.x;
+  uint32_t *own = reinterpret_cast<uint32_t *>(sweep_smem), *halo = own + W;
+  const bool rev = (int)blockIdx.x >= nb;
+  const int b = rev ? (int)blockIdx.x - nb : (int)blockIdx.x;
+  for (int w = tid; w < 2 * W; w += SWEEP_THREADS) own[w] = 0;
+  if (tid <= L.ncol) s_row[tid] = L.colour_row[tid];
+  if (tid < L.ncol + 2) s_cnt[tid] = 0;
+  __syncthreads();
+  for (int r = tid; r < L.n; r += SWEEP_THREADS)
+    if (block_of[r] == b) atomicOr(&own[r >> 5], 1u << (r & 31));
+  __syncthreads();
+  int entries = 0;
+  for (int step = 0; step < L.ncol; step++) {
+    const int c = rev ? step : L.ncol - 1 - step;
+    const int r0 = s_row[c], r1 = s_row[c + 1];
+    int cnt = 0;
+    for (int r = r0 + tid; r < r1; r += SWEEP_THREADS) {
+      if (!sweep_bit(own, r)) continue;
+      cnt++;
+      sweep_row(L, r, c, r0, [&](int j, int) {
+        entries++;
+        const bool earlier = rev ? j >= r1 : j < r0;
+        atomicOr(&(earlier ? own : halo)[j >> 5], 1u << (j & 31));
+      });
+    }
+    if (cnt) atomicAdd(&s_cnt[c], cnt);
+    __syncthreads();
+  }
+  int nh = 0;
+  uint32_t *out = bits + (size_t)blockIdx.x * 2 * W;
+  for (int w = tid; w < W; w += SWEEP_THREADS) {
+    const uint32_t o = own[w], h = halo[w] & ~o;
+    out[w] = o;
+    out[W + w] = h;
+    nh += __popc(h);
+  }
+  if (nh) atomicAdd(&s_cnt[L.ncol], nh);
+  if (entries) atomicAdd(&s_cnt[L.ncol + 1], entries);
+  __syncthreads();
+  if (tid < L.ncol + 2) counts[(size_t)blockIdx.x * (L.ncol + 2) + tid] = s_cnt[tid];
+}
+
+// the sets and their ranks into LDS (16 bytes per 32 rows)
+struct SweepSets {
+  uint32_t *own, *halo;
+  int *own_before, *halo_before;
+};
+__device__ __forceinline__ SweepSets sweep_sets(char *smem, int *part, int W, const uint32_t *bits) {
+  SweepSets s;
+  s.own = reinterpret_cast<uint32_t *>(smem);
+  s.halo = s.own + W;
+  s.own_before = reinterpret_cast<int *>(s.halo + W);
+  s.halo_before = s.own_before + W;
+  const uint32_t *in = bits + (size_t)blockIdx.x * 2 * W;
+  for (int w = threadIdx.x; w < 2 * W; w += SWEEP_THREADS) s.own[w] = in[w];
+  __syncthreads();
+  sweep_scan(W, part, [&](int w) { return __popc(s.own[w]); }, [&](int w, int v) { s.own_before[w] = v; });
+  sweep_scan(W, part, [&](int w) { return __popc(s.halo[w]); }, [&](int w, int v) { s.halo_before[w] = v; });
+  return s;
+}
+
+// the local rows, and the slices with their widths and offsets; a block's
+// n_ent.  Dynamic LDS: the sets, then max_slices widths
+__global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_rows(SweepLevel L, const int32_t *__restrict__ block_of, int nb,
+                                                              const uint32_t *__restrict__ bits,
+                                                              const int32_t *__restrict__ counts, int gs_fwd, int gs_rev,
+                                                              SweepBlock *__restrict__ blocks, int32_t *__restrict__ rows,
+                                                              SliceInfo *__restrict__ slices,
+                                                              int32_t *__restrict__ col_slice) {
+  extern __shared__ __align__(16) char sweep_smem[];
+  __shared__ int part[SWEEP_THREADS], s_row0[SWEEP_COLOURS + 1], s_slice0[SWEEP_COLOURS + 1];
+  const int W = (L.n + 31) / 32, tid = threadIdx.x, k = blockIdx.x;
+  const int b = k >= nb ? k - nb : k, gs = k >= nb ? gs_rev : gs_fwd, R = WAVE >> gs;
+  const SweepBlock B = blocks[k];
+  const SweepSets s = sweep_sets(sweep_smem, part, W, bits);
+  int *width = s.halo_before + W;
+  for (int w = tid; w < W; w += SWEEP_THREADS) {
+    int at = B.row0 + s.own_before[w];
+    for (uint32_t m = s.own[w]; m; m &= m - 1) {
+      const int r = w * 32 + __ffs((int)m) - 1;
+      rows[at++] = block_of[r] == b ? ~r : r;
+    }
+    at = B.row0 + B.n_rows + s.halo_before[w];
+    for (uint32_t m = s.halo[w]; m; m &= m - 1) rows[at++] = w * 32 + __ffs((int)m) - 1;
+  }
+  if (tid == 0) { // first local row and slice of each colour
+    int r = 0, q = 0;
+    for (int c = 0; c < L.ncol; c++) {
+      const int n = counts[(size_t)k * (L.ncol + 2) + c];
+      s_row0[c] = r;
+      s_slice0[c] = q;
+      r += n;
+      q += (n + R - 1) / R;
+    }
+    s_row0[L.ncol] = r;
+    s_slice0[L.ncol] = q;
+  }
+  for (int q = tid; q < B.n_slices; q += SWEEP_THREADS) width[q] = 0;
+  __syncthreads(); // the local rows are written, too
+  if (tid <= L.ncol) col_slice[(size_t)k * (L.ncol + 1) + tid] = s_slice0[tid];
+  for (int c = 0; c < L.ncol; c++) {
+    const int c_row0 = L.colour_row[c], n = s_row0[c + 1] - s_row0[c];
+    for (int i = tid; i < n; i += SWEEP_THREADS) {
+      const int v = rows[B.row0 + s_row0[c] + i];
+      int len = 0;
+      sweep_row(L, v < 0 ? ~v : v, c, c_row0, [&](int, int) { len++; });
+      atomicMax(&width[s_slice0[c] + i / R], (len + (1 << gs) - 1) >> gs);
+    }
+  }
+  __syncthreads();
+  for (int c = 0; c < L.ncol; c++) {
+    const int n = s_row0[c + 1] - s_row0[c];
+    for (int i = tid; i < (n + R - 1) / R; i += SWEEP_THREADS) {
+      SliceInfo &q = slices[B.slice0 + s_slice0[c] + i];
+      q.row0 = s_row0[c] + i * R;
+      q.nrow = n - i * R < R ? n - i * R : R;
+    }
+  }
+  const int steps = sweep_scan(
+      B.n_slices, part, [&](int q) { return width[q]; },
+      [&](int q, int v) {
+        slices[B.slice0 + q].width = width[q];
+        slices[B.slice0 + q].off = v * WAVE;
+      });
+  if (tid == 0) blocks[k].n_ent = steps * WAVE;
+}
+
+// the entries: local columns and positions in the level's layout (padding: a
+// local row, -1)
+__global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_entries(SweepLevel L, int nb, const uint32_t *__restrict__ bits,
+                                                                 int gs_fwd, int gs_rev,
+                                                                 const SweepBlock *__restrict__ blocks,
+                                                                 const int32_t *__restrict__ rows,
+                                                                 const SliceInfo *__restrict__ slices,
+                                                                 const int32_t *__restrict__ col_slice,
+                                                                 uint16_t *__restrict__ cols, int32_t *__restrict__ src) {
+  extern __shared__ __align__(16) char sweep_smem[];
+  __shared__ int part[SWEEP_THREADS];
+  const int W = (L.n + 31) / 32, k = blockIdx.x;
+  const int gs = k >= nb ? gs_rev : gs_fwd, R = WAVE >> gs, G = 1 << gs;
+  const SweepBlock B = blocks[k];
+  const SweepSets s = sweep_sets(sweep_smem, part, W, bits);
+  const int32_t *cs = col_slice + (size_t)k * (L.ncol + 1);
+  for (int c = 0; c < L.ncol; c++) {
+    const int c_row0 = L.colour_row[c], q0 = cs[c], lanes = (cs[c + 1] - q0) * R;
+    for (int i = threadIdx.x; i < lanes; i += SWEEP_THREADS) {
+      const SliceInfo q = slices[B.slice0 + q0 + i / R];
+      const int l = i % R, base = B.ent0 + q.off + (l << gs);
+      auto put = [&](int j, int col, int from) {
+        const int at = base + (j >> gs) * WAVE + (j & (G - 1));
+        cols[at] = (uint16_t)col;
+        src[at] = from;
+      };
+      int j = 0;
+      if (l < q.nrow) {
+        const int v = rows[B.row0 + q.row0 + l];
+        sweep_row(L, v < 0 ? ~v : v, c, c_row0, [&](int col, int pos) {
+          put(j++,
+              sweep_bit(s.own, col) ? sweep_rank(s.own, s.own_before, col)
+                                    : B.n_rows + sweep_rank(s.halo, s.halo_before, col),
+              pos);
+        });
+      }
+      for (; j < q.width << gs; j++) put(j, l < q.nrow ? q.row0 + l : 0, -1);
+    }
+  }
+}
+
 // the blocks' values from the level's layout (padding: 0)
+template <class T>
 __global__ __launch_bounds__(256) void k_sweep_values(int64_t n, const int32_t *__restrict__ src,
-                                                      const double *__restrict__ l64, double *__restrict__ v64,
-                                                      const float *__restrict__ l32, float *__restrict__ v32) {
+                                                      const T *__restrict__ level, T *__restrict__ v) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int32_t p = src[i];
-  v64[i] = p < 0 ? 0.0 : l64[p];
-  if (v32) v32[i] = p < 0 ? 0.0f : l32[p];
+  v[i] = p < 0 ? (T)0 : level[p];
 }
 
 // ---------------------------------------------------------------------------

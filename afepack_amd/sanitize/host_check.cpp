@@ -2,8 +2,8 @@
 // every element kind for a build with AddressSanitizer and
 // UndefinedBehaviorSanitizer: mesh generation, first-touch numbering with and
 // without side lists, the two-space pattern, both coarsenings (Project and
-// lazyProject), lazy refresh, colouring and the sliced-ELL layouts with
-// their source maps.  Exits 0 when every structural check holds.
+// lazyProject), lazy refresh, colouring, the sliced-ELL layouts with their
+// source maps, and the partitions of the block sweeps.  Exits 0 when every structural check holds.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -40,6 +40,8 @@ static Csr laplacian_on(const Space &s) {
   return A;
 }
 
+static void sweeps(const Csr &A, const std::vector<int32_t> &colour, int nc, int64_t target);
+
 static void layouts(const Hierarchy &h) {
   for (size_t l = 0; l < h.A.size(); l++) {
     const Csr &A = h.A[l];
@@ -48,6 +50,7 @@ static void layouts(const Hierarchy &h) {
     for (int64_t i = 0; i < A.m; i++)
       for (int64_t k = A.rp[i]; k < A.rp[i + 1]; k++)
         if (A.col[k] != i) CHECK(colour[i] != colour[A.col[k]]);
+    for (int64_t target : {1, 32, 100, 1000}) sweeps(A, colour, nc, target);
     std::vector<int32_t> perm(A.m), iperm(A.m), groups(nc, 0);
     for (int64_t i = 0; i < A.m; i++) groups[colour[i]]++;
     std::vector<int64_t> start(nc + 1, 0);
@@ -72,6 +75,69 @@ static void layouts(const Hierarchy &h) {
       build_sell(transpose(h.P[l]), perm, cperm, {(int32_t)A.m}, false, st);
       CHECK(sp.n_rows == nc1 && st.n_rows == A.m);
     }
+  }
+}
+
+// blocks of the sweeps: every row in one block, none empty, none beyond its
+// target by more than fragments; and a colour sweep by blocks, each updating
+// its rows' closure (neighbours of an earlier colour, and theirs) from the old
+// values of all others, is the colour sweep, bit for bit
+static void sweeps(const Csr &A, const std::vector<int32_t> &colour, int nc, int64_t target) {
+  std::vector<int32_t> block, order(A.m);
+  for (int64_t i = 0; i < A.m; i++) order[i] = (int32_t)(A.m - 1 - i);
+  const int nb = sweep_partition(A, target, order, block);
+  std::vector<int64_t> size(nb, 0);
+  CHECK((int64_t)block.size() == A.m);
+  for (int32_t b : block) {
+    CHECK(b >= 0 && b < nb);
+    size[b]++;
+  }
+  int64_t whole = 0;
+  for (int64_t s : size) {
+    CHECK(s > 0);
+    whole += s >= target;
+  }
+  CHECK(A.m >= target ? whole > 0 : nb >= 1);
+  std::vector<double> x0(A.m), rhs(A.m);
+  for (int64_t i = 0; i < A.m; i++) {
+    x0[i] = 0.001 * (double)(i * 37 % 101);
+    rhs[i] = 0.01 * (double)(i * 53 % 97);
+  }
+  auto update = [&](std::vector<double> &x, int64_t i) {
+    double s = 0.0;
+    for (int64_t k = A.rp[i] + 1; k < A.rp[i + 1]; k++) s += A.val[k] * x[A.col[k]];
+    x[i] = (rhs[i] - s) / A.val[A.rp[i]];
+  };
+  for (int rev = 0; rev <= 1; rev++) {
+    auto step = [&](int64_t i) { return rev ? nc - 1 - colour[i] : colour[i]; };
+    std::vector<double> want = x0, got(A.m, 0.0);
+    for (int c = 0; c < nc; c++)
+      for (int64_t i = 0; i < A.m; i++)
+        if (step(i) == c) update(want, i);
+    for (int b = 0; b < nb; b++) {
+      std::vector<int64_t> list;
+      std::vector<char> in(A.m, 0);
+      for (int64_t i = 0; i < A.m; i++)
+        if (block[i] == b) {
+          in[i] = 1;
+          list.push_back(i);
+        }
+      for (size_t h = 0; h < list.size(); h++)
+        for (int64_t k = A.rp[list[h]]; k < A.rp[list[h] + 1]; k++) {
+          const int64_t j = A.col[k];
+          if (!in[j] && step(j) < step(list[h])) {
+            in[j] = 1;
+            list.push_back(j);
+          }
+        }
+      std::vector<double> x = x0;
+      for (int c = 0; c < nc; c++)
+        for (int64_t i : list)
+          if (step(i) == c) update(x, i);
+      for (int64_t i = 0; i < A.m; i++)
+        if (block[i] == b) got[i] = x[i];
+    }
+    CHECK(got == want);
   }
 }
 

@@ -516,6 +516,13 @@ int afe_amg_device_info(const afe_amg *g, int32_t level, int64_t *rows,
                         int32_t *colours, int64_t *stored, int32_t *tail_level,
                         int32_t *row_lanes);
 
+/* sweeps of a level by independent blocks, one launch each (formed with the
+ * hierarchy's first own cycle): blocks per direction (0: one launch per
+ * colour), rows updated by the blocks of the forward [0] and the reverse [1]
+ * sweep, and whether FP64 [0] / FP32 [1] sweeps run so */
+int afe_amg_sweep_info(const afe_amg *g, int32_t level, int32_t *blocks,
+                       int64_t *updated, int32_t *fused);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,6 +1,6 @@
 """CPU: the host code of the library (csrc/host.cpp: numbering, patterns,
 two-space pattern, Project / lazyProject, Galerkin products, colouring,
-sliced-ELL layouts) and the oracle, built with AddressSanitizer and
+sliced-ELL layouts, block partitions of the sweeps) and the oracle, built with AddressSanitizer and
 UndefinedBehaviorSanitizer (afepack_amd/sanitize/Makefile) and run over small
 meshes of every element kind: no sanitizer report, no leak, and the drivers'
 own structural and convergence checks hold."""
