@@ -110,6 +110,7 @@ struct afe_ctx {
   double *d_bary = nullptr; // reference barycentrics of every rule point (same indexing)
   int64_t lds_bytes = 0;    // LDS granted to the coarse-tail workgroup
   std::map<void *, int64_t> user_bytes; // afe_dev_alloc buffers
+  int64_t most_bytes = 0; // bound on `bytes` for the library's own buffers (0: none)
   // device workspace of one call (call_scratch), kept between calls; used
   // with the context lock held and idle when the lock is released
   double *scratch = nullptr;
@@ -117,6 +118,9 @@ struct afe_ctx {
   bool keep_scratch = true;
   double *h_red = nullptr; // pinned: the result of a reduction, written by its kernel
 };
+
+// whether the context may hold `more` bytes in buffers of the library
+static bool has_room(const afe_ctx *c, int64_t more) { return c->most_bytes == 0 || c->bytes + more <= c->most_bytes; }
 
 // device bytes allocated minus freed by the calling thread (the server
 // measures what one request's set-up keeps)
@@ -179,8 +183,9 @@ template <class T> struct DevBuf {
     release();
     ctx = c;
     if (count == 0) return;
-    const hipError_t e = stream_ordered_alloc() ? hipMallocAsync((void **)&p, count * sizeof(T), c->stream)
-                                                : hipMalloc((void **)&p, count * sizeof(T));
+    const hipError_t e = !has_room(c, count * sizeof(T)) ? hipErrorOutOfMemory
+                         : stream_ordered_alloc()        ? hipMallocAsync((void **)&p, count * sizeof(T), c->stream)
+                                                         : hipMalloc((void **)&p, count * sizeof(T));
     if (e != hipSuccess) {
       p = nullptr;
       (void)hipGetLastError();
@@ -217,7 +222,7 @@ static double *call_scratch(afe_ctx *c, size_t n, DevBuf<double> &own) {
       c->scratch = nullptr;
       c->scratch_n = 0;
     }
-    if (hipMalloc((void **)&c->scratch, n * sizeof(double)) != hipSuccess) {
+    if (!has_room(c, n * sizeof(double)) || hipMalloc((void **)&c->scratch, n * sizeof(double)) != hipSuccess) {
       c->scratch = nullptr;
       (void)hipGetLastError();
       throw afe::Error{AFE_E_NOMEM, "device allocation of " + std::to_string(n * sizeof(double)) + " bytes failed"};
@@ -306,6 +311,9 @@ extern "C" int afe_ctx_create(int device, afe_ctx **out) {
   if (device < 0 || device >= n) return fail(AFE_E_NODEVICE, "device index out of range");
   auto *c = new afe_ctx();
   c->device = device;
+  // AFE_DEVICE_BYTES bounds what the library's own buffers of a context may
+  // take (the tests come to every shortage of memory through it)
+  if (const char *e = getenv("AFE_DEVICE_BYTES")) c->most_bytes = std::strtoll(e, nullptr, 10);
   HIPCHK(hipSetDevice(device));
   scratch_init(device);
   HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
@@ -1725,12 +1733,13 @@ struct afe_amg {
   DevBuf<double> minv;
   // the sub-cycle from dense_level down (from x = 0) as a matrix, for the
   // stationary [0] and the symmetric [1] cycle; nu: the smoothing count it was
-  // built for, -1 when the values or the coarse solve changed since
+  // built for, -1 when the values or the coarse solve changed since; off: there
+  // was no room for it since then
   int dense_level = -1;
-  bool dense_off = false; // its memory could not be allocated
   struct Dense {
     DevBuf<double> m;
     int nu = -1;
+    bool off = false;
   } dense[2];
   DevBuf<LevelDev<double>> ld64;
   DevBuf<LevelDev<float>> ld32;
@@ -1795,7 +1804,13 @@ static void alloc_pinned(afe_amg *g) {
   g->h_rr = reinterpret_cast<double *>(g->h_sc + 1);
 }
 
-static void drop_dense(afe_amg *g) { g->dense[0].nu = g->dense[1].nu = -1; }
+static void drop_dense(afe_amg *g) {
+  for (afe_amg::Dense &d : g->dense) {
+    if (d.off) drop_graphs(g); // captured without the matrix, which is tried again
+    d.nu = -1;
+    d.off = false;
+  }
+}
 
 // host CSR of the fine matrix (values from the device)
 static Csr fine_csr(afe_matrix *a) {
@@ -2087,10 +2102,10 @@ static void choose_dense_level(afe_amg *g) {
 // that runs the levels before it.  A cycle without smoothing has no colour
 // steps to save, and maps onto the coarsest space only, which the matrix's
 // rounding would leave.
-static bool dense_used(const afe_amg *g, int nu) {
+static bool dense_used(const afe_amg *g, bool symmetric, int nu) {
   const int ld = g->dense_level, Lc = (int)g->lv.size() - 1;
-  if (ld < 1 || nu == 0 || g->dense_off) return false;
-  if (ld < Lc) return true;
+  if (ld < 1 || nu == 0) return false;
+  if (ld < Lc) return !g->dense[symmetric ? 1 : 0].off;
   return g->coarse_mode == 0 && (g->tail0 == Lc || g->lv[Lc].n > COARSE_TAIL_MAX);
 }
 
@@ -2136,7 +2151,7 @@ static void build_dense(afe_amg *g, int ld, int lc, const double *minv, int coar
 // below, V(3,3): the first solve on new values 6.0 -> 3.6 ms).
 static void ensure_dense(afe_amg *g, bool symmetric, int nu) {
   const int ld = g->dense_level, Lc = (int)g->lv.size() - 1;
-  if (!dense_used(g, nu) || ld == Lc) return;
+  if (!dense_used(g, symmetric, nu) || ld == Lc) return;
   afe_amg::Dense &d = g->dense[symmetric ? 1 : 0];
   if (d.nu == nu) return;
   try {
@@ -2149,8 +2164,11 @@ static void ensure_dense(afe_amg *g, bool symmetric, int nu) {
     } else {
       build_dense(g, ld, Lc, g->minv.p, g->coarse_mode, symmetric, nu, d.m);
     }
-  } catch (const afe::Error &) { // no room: the levels stay as they are
-    g->dense_off = true;
+  } catch (const afe::Error &x) { // no room: the levels stay as they are until new values come
+    if (x.code != AFE_E_NOMEM) throw;
+    d.m.release();
+    d.nu = -1;
+    d.off = true;
     drop_graphs(g);
     return;
   }
@@ -3039,7 +3057,7 @@ static void gs_colour(DevLevel &d, int c, hipStream_t st) {
 template <class T>
 static void issue_vcycle(afe_amg *g, int nu, bool symmetric, hipStream_t st, bool x0_zero) {
   const int Lc = (int)g->lv.size() - 1;
-  const bool dense = dense_used(g, nu);
+  const bool dense = dense_used(g, symmetric, nu);
   // levels run as launches: those before the tail, or all before the dense
   // level when the ones between have one-launch sweeps (a level of 3692 rows:
   // two sweeps, residual and transfers 26 us, 50 us in the tail's two legs)
