@@ -2711,6 +2711,8 @@ static void device_lazy_refresh(afe_amg *g, afe_matrix *a) {
   hipStream_t s = ctx->stream;
   Hierarchy &h = g->h;
   const int L = (int)g->lv.size();
+  // first: a refresh that fails below leaves no matrix of older values
+  drop_dense(g);
   auto lvals = [&](int l) -> const double * { return l == 0 ? a->val.p : g->lv[l].c_val.p; };
   for (int l = 0; l + 1 < L; l++) {
     DevLevel &d = g->lv[l];
@@ -2756,7 +2758,6 @@ static void device_lazy_refresh(afe_amg *g, afe_matrix *a) {
   HIPCHK(hipStreamSynchronize(s));
   g->A0 = a;
   g->host_vals_stale = true;
-  drop_dense(g);
   retry_sweeps(g);
 }
 
