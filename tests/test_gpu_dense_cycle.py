@@ -78,3 +78,25 @@ def test_matrix_form_equals_the_steps(ctx, monkeypatch, kind, n, lazy, smooth, r
     for g in (g0, g1):
         g.set_coarse_exact(False)
     compare(ctx, g0, g1, sp.n_dof, rng)
+
+
+def test_what_a_solve_keeps(ctx):
+    """A solve's first cycle keeps the matrix and workspace for 512 columns of
+    three vectors on the levels down from it, not for all columns, beside the
+    sweep tables of a level of 4225 rows (below 4 MB)."""
+    import afepack_amd as afe
+    print("case dense workspace", flush=True)
+    c, ev, vm = make_mesh(1, 64, 0.05, 13)
+    own = afe.Context(0)
+    sp = afe.Space(own, 1, c, ev, vm)
+    A = afe.Matrix(sp)
+    A.assemble(afe.OP_STIFF, 4)
+    b = sp.rhs(4, afe.F_POISSON)
+    A.apply_dirichlet(b)
+    g = afe.Amg(A, afe.AmgParams(lazy=0, smooth=3, build_fp32=0))
+    x = afe.DeviceVector(own, sp.n_dof)
+    held = own.device_bytes()
+    g.solve(x, b)
+    n = g.info()["n"]
+    assert 512 < n[1] <= 2560
+    assert own.device_bytes() - held <= 8 * n[1] ** 2 + 512 * 3 * 8 * sum(n[1:]) + (4 << 20)
