@@ -127,6 +127,7 @@ SIGS = {
     "afe_batch_set_tiles": (C.c_int, [P, I32, I32]),
     "afe_amg_device_info": (C.c_int, [P, I32, PI64, PI32, PI64, PI32, PI32]),
     "afe_amg_sweep_info": (C.c_int, [P, I32, PI32, PI64, PI32]),
+    "afe_amg_dense_info": (C.c_int, [P, PI32, PI32]),
 }
 
 

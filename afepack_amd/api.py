@@ -558,6 +558,13 @@ class Amg(_AmgBase):
                         "row_lanes": g.value})
         return out
 
+    def dense_info(self):
+        """first level of the sub-cycle applied as a matrix (-1: none), and whether the (stationary, symmetric)
+        cycle applies it now"""
+        l, f = C.c_int32(), (C.c_int32 * 2)()
+        _chk(_lib().afe_amg_dense_info(self.h, C.byref(l), f))
+        return l.value, (bool(f[0]), bool(f[1]))
+
     def sweep_info(self):
         """per level: blocks of the one-launch sweeps (0: none), rows they update (forward, reverse), fused in
         (FP64, FP32)"""

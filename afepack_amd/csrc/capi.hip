@@ -1734,12 +1734,14 @@ struct afe_amg {
   // the sub-cycle from dense_level down (from x = 0) as a matrix, for the
   // stationary [0] and the symmetric [1] cycle; nu: the smoothing count it was
   // built for, -1 when the values or the coarse solve changed since; off: there
-  // was no room for it since then
+  // was no room for it since then; steps: cycles run without it since then, of
+  // smoothing count steps_nu
   int dense_level = -1;
   struct Dense {
     DevBuf<double> m;
     int nu = -1;
     bool off = false;
+    int steps = 0, steps_nu = -1;
   } dense[2];
   DevBuf<LevelDev<double>> ld64;
   DevBuf<LevelDev<float>> ld32;
@@ -1766,37 +1768,35 @@ struct afe_amg {
   // the levels' sweep tables (as far as they have any), and their values per
   // precision; short: there was no room for some
   bool sweeps_formed = false, sweeps_ready[2] = {false, false}, sweeps_short = false;
-  // captured V-cycles: [precision][symmetric]
-  hipGraphExec_t vc_graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
-  // captured CG iteration in two parts: [part][precision]; part 0 ends with
-  // the copy of the scalars to the host, part 1 is the preconditioner and the
-  // direction update
-  hipGraphExec_t cg_graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
-  int graph_nu[2][2] = {{-1, -1}, {-1, -1}};
-  int cg_nu[2][2] = {{-1, -1}, {-1, -1}};
+  struct Graph {
+    hipGraphExec_t ex = nullptr;
+    int nu = -1;
+  };
+  // captured V-cycles: [precision][symmetric][with the sub-cycle's matrix]
+  Graph vc_graph[2][2][2];
+  // captured CG iteration in two parts: [part][precision][with the matrix];
+  // part 0 ends with the copy of the scalars to the host, part 1 is the
+  // preconditioner and the direction update
+  Graph cg_graph[2][2][2];
   hipEvent_t it_ev = nullptr; // recorded after part 0 of each CG iteration
 };
 
 static void drop_graphs(afe_amg *g) {
+  auto all = [&](auto f) {
+    for (auto *set : {&g->vc_graph, &g->cg_graph})
+      for (auto &a : *set)
+        for (auto &b : a)
+          for (afe_amg::Graph &e : b)
+            if (e.ex) f(e);
+  };
   bool any = false;
-  for (auto &row : g->vc_graph)
-    for (auto &e : row) any = any || e;
-  for (auto &row : g->cg_graph)
-    for (auto &e : row) any = any || e;
+  all([&](afe_amg::Graph &) { any = true; });
   // no executable graph is destroyed while a launch of it may still run
   if (any && g->ctx) (void)hipStreamSynchronize(g->ctx->stream);
-  for (auto &row : g->vc_graph)
-    for (auto &e : row)
-      if (e) {
-        (void)hipGraphExecDestroy(e);
-        e = nullptr;
-      }
-  for (auto &row : g->cg_graph)
-    for (auto &e : row)
-      if (e) {
-        (void)hipGraphExecDestroy(e);
-        e = nullptr;
-      }
+  all([&](afe_amg::Graph &e) {
+    (void)hipGraphExecDestroy(e.ex);
+    e.ex = nullptr;
+  });
 }
 
 static void alloc_pinned(afe_amg *g) {
@@ -1806,9 +1806,9 @@ static void alloc_pinned(afe_amg *g) {
 
 static void drop_dense(afe_amg *g) {
   for (afe_amg::Dense &d : g->dense) {
-    if (d.off) drop_graphs(g); // captured without the matrix, which is tried again
-    d.nu = -1;
+    d.nu = d.steps_nu = -1;
     d.off = false;
+    d.steps = 0;
   }
 }
 
@@ -2075,7 +2075,7 @@ static void set_coarse_mode(afe_amg *g) {
 // in the single-workgroup tail, while the product with its matrix is one
 // launch: 2213^2 entries, 39 MB, 9 us.  Building it takes the tail's time once
 // per 256 columns (and again after new values), so the line lies where one
-// solve still gains: 21 stationary cycles on 4225 DOFs 11.4 ms without the
+// solve still gains (DENSE_CYCLES is the line of shorter calls): 21 stationary cycles on 4225 DOFs 11.4 ms without the
 // matrix, 4.9 / 3.1 / 1.7 ms with levels of up to 600 / 1100 / 2560 rows in it;
 // a moving-mesh step of 251K DOFs (refresh, matrix and 30 CG iterations) 9.30,
 // 8.71 / 8.05 / 8.03 ms, and 8.72 with 5000 rows.
@@ -2097,6 +2097,17 @@ static void choose_dense_level(afe_amg *g) {
     }
 }
 
+// The matrix is formed when at least this many cycles with the same values and
+// smoothing count have run without it or may still run in the call at hand (a
+// solve counts with its bound): forming it takes as long as it saves in 2 to 5
+// cycles.  A program that changes the values and then applies one cycle, or
+// switches between smoothing counts, runs the levels step by step.  1 / 3 / 10
+// FP64 V(1,1) cycles after a refresh, the matrix formed with the first cycle and
+// by this rule: 251K P1 DOFs 0.42 / 0.77 / 1.94 and 0.26 / 0.75 / 2.18 ms, 58K P2
+// 0.35 / 0.55 / 1.25 and 0.15 / 0.45 / 1.39, 373K of tetrahedra 0.62 / 1.44 / 4.31
+// and 0.53 / 1.48 / 4.53.
+constexpr int DENSE_CYCLES = 4;
+
 // whether cycles apply dense_level as a matrix.  When that is the coarsest
 // level its matrix is the dense inverse; a small one stays inside the tail
 // that runs the levels before it.  A cycle without smoothing has no colour
@@ -2105,7 +2116,7 @@ static void choose_dense_level(afe_amg *g) {
 static bool dense_used(const afe_amg *g, bool symmetric, int nu) {
   const int ld = g->dense_level, Lc = (int)g->lv.size() - 1;
   if (ld < 1 || nu == 0) return false;
-  if (ld < Lc) return !g->dense[symmetric ? 1 : 0].off;
+  if (ld < Lc) return g->dense[symmetric ? 1 : 0].nu == nu;
   return g->coarse_mode == 0 && (g->tail0 == Lc || g->lv[Lc].n > COARSE_TAIL_MAX);
 }
 
@@ -2150,16 +2161,21 @@ static void build_dense(afe_amg *g, int ld, int lc, const double *minv, int coar
   HIPCHK(hipStreamSynchronize(st)); // before the tables go
 }
 
-// builds the matrix of the sub-cycle if it is used and not current.  In two
-// steps when a level of at most COARSE_TAIL_MAX rows lies further down: that
+// before a cycle, with `ahead` cycles that the call may still run, this one
+// included: forms the matrix of the sub-cycle if it is not current and pays.  In
+// two steps when a level of at most COARSE_TAIL_MAX rows lies further down: that
 // level's matrix first, in one round of workgroups, which then is the coarse
 // solve of all the other columns (2213 rows with levels of 692, 227, 81 and 33
 // below, V(3,3): the first solve on new values 6.0 -> 3.6 ms).
-static void ensure_dense(afe_amg *g, bool symmetric, int nu) {
+static void ensure_dense(afe_amg *g, bool symmetric, int nu, int64_t ahead) {
   const int ld = g->dense_level, Lc = (int)g->lv.size() - 1;
-  if (!dense_used(g, symmetric, nu) || ld == Lc) return;
   afe_amg::Dense &d = g->dense[symmetric ? 1 : 0];
-  if (d.nu == nu) return;
+  if (ld < 1 || ld == Lc || nu == 0 || d.nu == nu || d.off) return;
+  if (d.steps_nu != nu) {
+    d.steps_nu = nu;
+    d.steps = 0;
+  }
+  if (d.steps + ahead < DENSE_CYCLES) return;
   try {
     int lc = ld + 1;
     while (lc < Lc && g->lv[lc].n > COARSE_TAIL_MAX) lc++;
@@ -2179,6 +2195,12 @@ static void ensure_dense(afe_amg *g, bool symmetric, int nu) {
     return;
   }
   d.nu = nu;
+}
+
+// after the launch of a cycle
+static void count_cycle(afe_amg *g, bool symmetric, int nu) {
+  afe_amg::Dense &d = g->dense[symmetric ? 1 : 0];
+  if (d.nu != nu && d.steps < DENSE_CYCLES) d.steps++;
 }
 
 // Levels whose sweeps run as one launch: of at most SWEEP_ROWS rows (larger
@@ -3197,9 +3219,11 @@ static bool use_graphs() {
   return v;
 }
 
-static void launch_graph_or_issue(afe_amg *g, int prec, bool symmetric, int nu) {
+// one cycle; ahead: the cycles that the call may still run, this one included
+static void launch_graph_or_issue(afe_amg *g, int prec, bool symmetric, int nu, int64_t ahead) {
   hipStream_t st = g->ctx->stream;
-  ensure_dense(g, symmetric, nu);
+  ensure_dense(g, symmetric, nu, ahead);
+  count_cycle(g, symmetric, nu);
   if (prec == 1) ensure_sweeps<float>(g, nu);
   else ensure_sweeps<double>(g, nu);
   if (!use_graphs()) {
@@ -3213,23 +3237,22 @@ static void launch_graph_or_issue(afe_amg *g, int prec, bool symmetric, int nu) 
     drop_graphs(g);
     g->graph_epoch = g_tune.epoch;
   }
-  hipGraphExec_t &ex = g->vc_graph[prec][symmetric ? 1 : 0];
-  if (ex && g->graph_nu[prec][symmetric ? 1 : 0] != nu) {
-    (void)hipGraphExecDestroy(ex);
-    ex = nullptr;
+  afe_amg::Graph &e = g->vc_graph[prec][symmetric ? 1 : 0][dense_used(g, symmetric, nu) ? 1 : 0];
+  if (e.ex && e.nu != nu) {
+    (void)hipGraphExecDestroy(e.ex);
+    e.ex = nullptr;
   }
-  if (!ex) {
-    ex = capture_graph(st, [&]() {
+  if (!e.ex) {
+    e.ex = capture_graph(st, [&]() {
       if (prec == 1)
         issue_vcycle<float>(g, nu, symmetric, st, symmetric);
       else
         issue_vcycle<double>(g, nu, symmetric, st, symmetric);
     });
-    g->graph_nu[prec][symmetric ? 1 : 0] = nu;
+    e.nu = nu;
   }
-  HIPCHK(hipGraphLaunch(ex, st));
+  HIPCHK(hipGraphLaunch(e.ex, st));
 }
-
 
 // true residual r = b - A (x + xl) in compensated arithmetic, and its norms
 // natural = true: vectors in the natural numbering (the CG), else in the
@@ -3277,14 +3300,14 @@ extern "C" int afe_amg_solve(afe_amg *g, double *d_x, const double *d_r, double 
   if (rtol <= 0 && !(mode & 2) && !verbose()) {
     // the reference's form (no early exit, nothing printed per cycle): the
     // step + 1 cycles run back to back, the residual is taken once after them
-    for (; it <= step; it++) launch_graph_or_issue(g, 0, false, g->prm.smooth);
+    for (; it <= step; it++) launch_graph_or_issue(g, 0, false, g->prm.smooth, step + 1 - it);
     residual_norms(g, false, d0.b64.p, d0.x64.p, nullptr);
     read_scalars(g);
     rr = g->h_sc->rr;
     l1 = g->h_sc->l1;
   } else {
     while (true) {
-      launch_graph_or_issue(g, 0, false, g->prm.smooth);
+      launch_graph_or_issue(g, 0, false, g->prm.smooth, step + 1 - it);
       residual_norms(g, false, d0.b64.p, d0.x64.p, nullptr);
       read_scalars(g);
       rr = g->h_sc->rr;
@@ -3336,12 +3359,12 @@ constexpr int CG_SUM_PARTIALS = 4096;
 
 // z = M^{-1} r with one symmetric V-cycle from zero; r and z in the natural
 // numbering, the V-cycle in the level-0 colour order
-template <class T> static void precondition_perm(afe_amg *g, const double *r, bool first) {
+template <class T> static void precondition_perm(afe_amg *g, const double *r, bool first, int ahead) {
   DevLevel &d0 = g->lv[0];
   hipStream_t s = g->ctx->stream;
   const int64_t n = d0.n;
   k_prep_vcycle<T><<<nblk(n), 256, 0, s>>>(n, r, Prec<T>::b(d0), Prec<T>::x(d0), g->iperm0.p);
-  launch_graph_or_issue(g, std::is_same<T, float>::value ? 1 : 0, true, g->prm.smooth);
+  launch_graph_or_issue(g, std::is_same<T, float>::value ? 1 : 0, true, g->prm.smooth, ahead);
   if (first) k_fill<double><<<nblk(n), 256, 0, s>>>(n, g->wz.p, 0.0);
   const unsigned nb = cg_blocks(n);
   k_take_z<T><<<nb, 256, 0, s>>>(n, Prec<T>::x(d0), r, g->wz.p, g->iperm0.p, g->part.p);
@@ -3415,16 +3438,16 @@ template <class F> static void launch_part(afe_amg *g, int part, int prec, F iss
     drop_graphs(g);
     g->graph_epoch = g_tune.epoch;
   }
-  hipGraphExec_t &ex = g->cg_graph[part][prec];
-  if (ex && g->cg_nu[part][prec] != g->prm.smooth) {
-    (void)hipGraphExecDestroy(ex);
-    ex = nullptr;
+  afe_amg::Graph &e = g->cg_graph[part][prec][dense_used(g, true, g->prm.smooth) ? 1 : 0];
+  if (e.ex && e.nu != g->prm.smooth) {
+    (void)hipGraphExecDestroy(e.ex);
+    e.ex = nullptr;
   }
-  if (!ex) {
-    ex = capture_graph(st, issue);
-    g->cg_nu[part][prec] = g->prm.smooth;
+  if (!e.ex) {
+    e.ex = capture_graph(st, issue);
+    e.nu = g->prm.smooth;
   }
-  HIPCHK(hipGraphLaunch(ex, st));
+  HIPCHK(hipGraphLaunch(e.ex, st));
 }
 
 // one CG iteration: part 0 (with the SpMV; with live timing the SpMV is
@@ -3446,6 +3469,7 @@ template <class T> static void launch_cg_iteration(afe_amg *g) {
   HIPCHK(hipEventRecord(g->it_ev, st));
   if (pe) HIPCHK(hipEventRecord(pe[1], st));
   launch_part(g, 1, prec, [&]() { issue_cg_precondition<T>(g); });
+  count_cycle(g, true, g->prm.smooth);
   if (pe) HIPCHK(hipEventRecord(pe[2], st));
 }
 
@@ -3497,7 +3521,7 @@ static int pcg_impl(afe_amg *g, double *d_x, const double *d_b, double rtol, int
   for (int outer = 0; outer < 4; outer++) {
   while (!conv && it < max_it) {
     k_fill<double><<<nblk(n), 256, 0, s>>>(n, g->wp.p, 0.0);
-    precondition_perm<T>(g, g->wr.p, true);
+    precondition_perm<T>(g, g->wr.p, true, max_it - it + 1);
     while (it < max_it) {
       launch_cg_iteration<T>(g);
       HIPCHK(hipEventSynchronize(g->it_ev));
@@ -3590,11 +3614,11 @@ extern "C" int afe_amg_vcycle(afe_amg *g, double *d_z, const double *d_r, int32_
   k_permute_in<double, double><<<nblk(n), 256, 0, s>>>(n, g->perm0.p, d_r, g->wr.p);
   if (prec == AFE_PREC_FP32) {
     k_prep_vcycle<float><<<nblk(n), 256, 0, s>>>(n, g->wr.p, d0.b32.p, d0.x32.p, nullptr);
-    launch_graph_or_issue(g, 1, true, g->prm.smooth);
+    launch_graph_or_issue(g, 1, true, g->prm.smooth, 1);
     k_permute_out<float, double><<<nblk(n), 256, 0, s>>>(n, g->perm0.p, d0.x32.p, d_z);
   } else {
     k_prep_vcycle<double><<<nblk(n), 256, 0, s>>>(n, g->wr.p, d0.b64.p, d0.x64.p, nullptr);
-    launch_graph_or_issue(g, 0, true, g->prm.smooth);
+    launch_graph_or_issue(g, 0, true, g->prm.smooth, 1);
     k_permute_out<double, double><<<nblk(n), 256, 0, s>>>(n, g->perm0.p, d0.x64.p, d_z);
   }
   HIPCHK(hipStreamSynchronize(s));
@@ -3776,6 +3800,17 @@ extern "C" int afe_amg_device_info(const afe_amg *g, int32_t level, int64_t *row
   if (stored) *stored = (int64_t)d.cols.n;
   if (tail_level) *tail_level = g->tail0;
   if (row_lanes) *row_lanes = 1 << d.gs;
+  return AFE_OK;
+}
+
+// the small levels' sub-cycle as a matrix: the first level in it (-1: none) and
+// whether the stationary [0] / the symmetric [1] cycle has its matrix formed for
+// the current values and smoothing count
+extern "C" int afe_amg_dense_info(const afe_amg *g, int32_t *level, int32_t *formed) {
+  if (!g || !g->ctx) return fail(AFE_E_ARG, "bad arguments");
+  if (level) *level = g->dense_level;
+  if (formed)
+    for (int k = 0; k < 2; k++) formed[k] = g->dense_level > 0 && dense_used(g, k == 1, g->prm.smooth);
   return AFE_OK;
 }
 

@@ -516,6 +516,11 @@ int afe_amg_device_info(const afe_amg *g, int32_t level, int64_t *rows,
                         int32_t *colours, int64_t *stored, int32_t *tail_level,
                         int32_t *row_lanes);
 
+/* the cycle of the small levels as one matrix: its first level (-1: none), and
+ * whether the stationary [0] / the symmetric [1] cycle applies it now (it is
+ * formed for solves, and after a few single cycles on the same values) */
+int afe_amg_dense_info(const afe_amg *g, int32_t *level, int32_t *formed);
+
 /* sweeps of a level by independent blocks, one launch each (formed with the
  * hierarchy's first own cycle): blocks per direction (0: one launch per
  * colour), rows updated by the blocks of the forward [0] and the reverse [1]

@@ -3,7 +3,8 @@ run step by step (AFE_DENSE_ROWS=0): the symmetric and the stationary cycle,
 one and three sweeps, coarsest level solved by the inverse or smoothed, a
 hierarchy whose every level below the first is in the matrix, one with tail
 levels above it and one with the tail off; then after new values, after another
-smoothing count and after the coarse solve changes.
+smoothing count and after the coarse solve changes.  Which cycles form the
+matrix: solves, and the fourth single one on the same values and smoothing count.
 
 The matrix is the FP64 cycle's: FP64 results differ by rounding in sums of at
 most a few thousand terms (1e-12 relative bounds them, as in the other cycle
@@ -31,13 +32,14 @@ def compare(ctx, g0, g1, n, rng, f32=True):
     r = afe.DeviceVector.from_numpy(ctx, rng.uniform(-1, 1, n))
     z = [afe.DeviceVector(ctx, n) for _ in range(2)]
     for prec, tol in ((afe.PREC_FP64, 1e-12), (afe.PREC_FP32, 1e-5)):
-        for g, v in zip((g0, g1), z):
-            g.vcycle(v, r, prec)
-        a, b = (v.numpy() for v in z)
-        assert np.linalg.norm(a - b) <= tol * np.linalg.norm(a), prec
+        for _ in range(4):  # the matrix is formed by the fourth cycle at the latest
+            for g, v in zip((g0, g1), z):
+                g.vcycle(v, r, prec)
+            a, b = (v.numpy() for v in z)
+            assert np.linalg.norm(a - b) <= tol * np.linalg.norm(a), prec
     for g, v in zip((g0, g1), z):
         v.zero()
-        g.precondition(v, r, 2)  # three stationary cycles
+        g.precondition(v, r, 3)  # four stationary cycles
     a, b = (v.numpy() for v in z)
     assert np.linalg.norm(a - b) <= 1e-12 * np.linalg.norm(a)
 
@@ -59,7 +61,16 @@ def test_matrix_form_equals_the_steps(ctx, monkeypatch, kind, n, lazy, smooth, r
     for g in (g0, g1):
         g.set_tail_rows(tail)
     rng = np.random.default_rng(n)
-    compare(ctx, g0, g1, sp.n_dof, rng)
+    # the coarsest level alone: its matrix is the coarse solve's inverse
+    lone = g1.dense_info()[0] == g1.info()["levels"] - 1
+
+    def compare_formed():
+        compare(ctx, g0, g1, sp.n_dof, rng)
+        assert g0.dense_info() == (-1, (False, False))
+        assert g1.dense_info()[0] > 0
+        assert lone or g1.dense_info()[1] == (True, True)
+
+    compare_formed()
     xs = []
     for g in (g0, g1):
         x = afe.DeviceVector(ctx, sp.n_dof)
@@ -71,13 +82,63 @@ def test_matrix_form_equals_the_steps(ctx, monkeypatch, kind, n, lazy, smooth, r
         A.apply_dirichlet(b)
         for g in (g0, g1):
             g.lazy_reinit(A)
-        compare(ctx, g0, g1, sp.n_dof, rng)
+        compare_formed()
     for g in (g0, g1):
         g.set_smooth(2)
-    compare(ctx, g0, g1, sp.n_dof, rng)
+    compare_formed()
     for g in (g0, g1):
         g.set_coarse_exact(False)
-    compare(ctx, g0, g1, sp.n_dof, rng)
+    compare_formed()
+
+
+def test_which_cycles_form_the_matrix(ctx):
+    import afepack_amd as afe
+    print("case dense forming", flush=True)
+    c, ev, vm = make_mesh(1, 40, 0.05, 13)
+    sp = afe.Space(ctx, 1, c, ev, vm)
+    A = afe.Matrix(sp)
+    A.assemble(afe.OP_STIFF, 2)
+    b = sp.rhs(2, afe.F_POISSON)
+    A.apply_dirichlet(b)
+    g = afe.Amg(A, afe.AmgParams(lazy=1, smooth=1, build_fp32=1))
+    x = afe.DeviceVector(ctx, sp.n_dof)
+
+    def formed():
+        return g.dense_info()[1]
+
+    for _ in range(3):  # new values, then three cycles each time
+        for _ in range(3):
+            g.vcycle(x, b, afe.PREC_FP32)
+        x.zero()
+        g.precondition(x, b, 2)
+        assert formed() == (False, False)
+        g.lazy_reinit(A)
+    for k in range(4):  # either precision counts
+        assert formed() == (False, False)
+        g.vcycle(x, b, afe.PREC_FP64 if k % 2 else afe.PREC_FP32)
+    assert formed() == (False, True)
+    x.zero()
+    g.precondition(x, b, 3)
+    assert formed() == (True, True)
+    g.set_smooth(2)  # another count: three cycles of it, then back to the matrix
+    for _ in range(3):
+        g.vcycle(x, b, afe.PREC_FP64)
+    assert formed() == (False, False)
+    g.set_smooth(1)
+    assert formed() == (True, True)
+    g.lazy_reinit(A)
+    assert formed() == (False, False)
+    x.zero()
+    g.pcg(x, b, rtol=1e-8, max_it=100, prec=afe.PREC_FP32)
+    assert formed() == (False, True)
+    # the step form and the matrix agree along one call's cycles (captured both ways)
+    ref = afe.DeviceVector(ctx, sp.n_dof)
+    g.vcycle(ref, b, afe.PREC_FP64)
+    for _ in range(2):
+        g.lazy_reinit(A)
+        for k in range(6):
+            g.vcycle(x, b, afe.PREC_FP64)
+            assert np.linalg.norm(x.numpy() - ref.numpy()) <= 1e-12 * np.linalg.norm(ref.numpy())
 
 
 def test_what_a_solve_keeps(ctx):
