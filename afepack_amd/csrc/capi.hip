@@ -3407,7 +3407,10 @@ template <class T> static void issue_cg_update(afe_amg *g) {
                                                g->tail0 > 0 ? nullptr : Prec<T>::x(d0), g->iperm0.p, g->h_rr);
 }
 
-// (r, r) of the iteration whose part 0 has completed, in block order
+// (r, r) of the iteration whose part 0 has completed, in block order: at most
+// RED_BLOCKS sums of squares one after the other, within 1023 roundings (1.1e-13
+// relative) of their sum.  It decides when the iteration stops; what the solve
+// delivers is checked against the compensated true residual after it.
 static double cg_rr(const afe_amg *g) {
   double rr = 0.0;
   for (unsigned k = 0; k < cg_blocks(g->lv[0].n); k++) rr += g->h_rr[k];
@@ -3660,9 +3663,7 @@ extern "C" int afe_amg_kernel_timing(afe_amg *g, int32_t which, int32_t reps, do
   }
   auto once = [&]() {
     if (which == 0) {
-      k_spmv_dot<<<g_tune.spmv_blocks, BLK, 0, s>>>(g->nat_si.p, g->nat_ns, g->nat_cols.p, g->nat_c16.p,
-                                                     g->nat_cbase.p, g->nat_v64.p, g->nat_diag.p, g->nat_rowmap.p,
-                                                     g->wp.p, g->wq.p, g->part.p, g_tune.xcd);
+      issue_cg_spmv(g, s);
     } else if (which == 1) {
       for (int c = 0; c < d.ncol; c++) gs_colour<float>(d, c, s);
     } else if (which == 2) {

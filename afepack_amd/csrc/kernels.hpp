@@ -2086,8 +2086,8 @@ __global__ __launch_bounds__(256) void k_permute_out(int64_t n, const int32_t *_
   if (i < n) dst[perm[i]] = (D)src[i];
 }
 
-// y = A x (FP64, level 0) and the partial dots (x, y) per block; grid-stride
-// over slices with a fixed grid so the partial count is RED_BLOCKS
+// y = A x (FP64, level 0) and the partial dots (x, y), one per block of the
+// grid, which strides over the slices
 __global__ __launch_bounds__(BLK) void k_spmv_dot(const SliceInfo *__restrict__ si, int ns,
                                                   const int32_t *__restrict__ cols,
                                                   const uint16_t *__restrict__ c16,
