@@ -1334,8 +1334,9 @@ extern "C" int afe_matrix_tvmult(afe_matrix *a, const double *d_x, double *d_y) 
   if (!a || !d_x || !d_y) return fail(AFE_E_ARG, "null argument");
   std::lock_guard<CtxMutex> lk(a->ctx->mu);
   HIPCHK(hipSetDevice(a->ctx->device));
-  const bool wide = a->nnz > INT32_MAX;
   if (!a->t_ptr.p) {
+    // AFE_POS64=1 takes 64-bit positions at any size (both widths are tested)
+    const bool wide = a->nnz > INT32_MAX || getenv("AFE_POS64") != nullptr;
     // transposed index map of the pattern, built once per matrix
     std::vector<int64_t> tptr, tk;
     std::vector<int32_t> trow, tk32;
@@ -1354,7 +1355,7 @@ extern "C" int afe_matrix_tvmult(afe_matrix *a, const double *d_x, double *d_y) 
     kern<<<csr_grid(a->n), 256, 0, a->ctx->stream>>>(a->n, a->t_ptr.p, a->t_row.p, tk, a->val.p, d_x, d_y);
   };
   const bool staged = a->nnz <= CSR_LONG_ROWS * a->n;
-  if (wide)
+  if (a->t_k.p)
     staged ? go(k_csr_tvmult<true, int64_t>, a->t_k.p) : go(k_csr_tvmult<false, int64_t>, a->t_k.p);
   else
     staged ? go(k_csr_tvmult<true, int32_t>, a->t_k32.p) : go(k_csr_tvmult<false, int32_t>, a->t_k32.p);

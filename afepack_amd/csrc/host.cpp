@@ -399,6 +399,7 @@ void transpose_map(int64_t m, int64_t n, const std::vector<int64_t> &rp, const s
   for (int64_t j = 0; j < n; j++) tptr[j + 1] += tptr[j];
   trow.resize(nnz);
   tk.resize(nnz);
+  std::vector<int64_t> fill(tptr.begin(), tptr.end() - 1); // here: no allocation may fail in a thread
 #pragma omp parallel
   {
     const int64_t T = omp_get_num_threads(), t = omp_get_thread_num();
@@ -406,12 +407,11 @@ void transpose_map(int64_t m, int64_t n, const std::vector<int64_t> &rp, const s
       return s == T ? n : std::lower_bound(tptr.begin(), tptr.end(), nnz * s / T) - tptr.begin();
     };
     const int64_t j0 = bound(t), j1 = bound(t + 1);
-    std::vector<int64_t> fill(tptr.begin() + j0, tptr.begin() + std::max(j0, j1));
     for (int64_t i = 0; i < m && j0 < j1; i++)
       for (int64_t k = rp[i]; k < rp[i + 1]; k++) {
         const int64_t j = col[k];
         if (j < j0 || j >= j1) continue;
-        const int64_t p = fill[j - j0]++;
+        const int64_t p = fill[j]++;
         trow[p] = (int32_t)i;
         tk[p] = (K)k;
       }

@@ -19,7 +19,7 @@ def _matrix(m, lens, rng):
 
 @pytest.mark.parametrize("m,lens", [(1, 1), (255, 3), (256, 8), (257, 8), (600, 64), (520, 65), (300, 300),
                                     (700, "one long"), (1000, "mixed")])
-def test_products_are_the_sequential_sums(ctx, m, lens):
+def test_products_are_the_sequential_sums(ctx, monkeypatch, m, lens):
     import afepack_amd as afe
     print(f"case products m={m} lens={lens}", flush=True)
     rng = np.random.default_rng(m)
@@ -47,3 +47,8 @@ def test_products_are_the_sequential_sums(ctx, m, lens):
     for _ in range(2):  # the map is built by the first call
         A.tvmult(dx, dy)
         assert np.array_equal(dy.numpy(), yt)
+    # 64-bit positions, which matrices of 2^31 entries and more take
+    monkeypatch.setenv("AFE_POS64", "1")
+    B = afe.Matrix(ctx=ctx, csr=(rp, col, val))
+    B.tvmult(dx, dy)
+    assert np.array_equal(dy.numpy(), yt)
