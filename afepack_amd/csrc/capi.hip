@@ -1268,32 +1268,40 @@ extern "C" double *afe_matrix_device_values(afe_matrix *a) { return a ? a->val.p
 // XCDs in contiguous ranges: neighbouring rows gather the same x (and, in the
 // transposed product, entries of the same rows) through one L2.  HBM bound.
 // 1.05M P2 DOFs, 12.1M entries: vmult 223 -> 44 us (3.5 TB/s), Tvmult 353 ->
-// 55 us, both with one thread walking its row before.  That form stays for
-// rows of more than CSR_LONG_ROWS entries on average: a chunk then holds few
-// rows, and most threads wait for their serial sums.  4M entries in rows of
-// 64: 65 us staged, 80 walking; of 96: 100 and 63; of 1024: 5.8 ms and 0.41.
+// 55 us, both with one thread walking its row before.  A block of long rows
+// walks them still: a chunk then holds few rows, and most threads wait for their
+// serial sums.  Staged, a block takes 43 ns for each entry of its longest row in
+// a chunk, walking 170 to 450 ns for each entry of its longest row, so the line
+// is CSR_WALK times the longest row, or times a chunk where no row fills one.  4M
+// entries in rows of 64: 65 us staged, 80 walking; of 96: 100 and 63; of 1024:
+// 5.8 ms and 0.41.  Among 200K rows of 7, one of 100K entries: 4.4 ms and 17; 10
+// of them together 43 and 18; 256 rows of 10K together 79 and 4.5.
 #pragma clang fp contract(off)
-constexpr int CSR_ROWS = 256, CSR_CHUNK = 2048, CSR_LONG_ROWS = 64;
+constexpr int CSR_ROWS = 256, CSR_CHUNK = 2048, CSR_WALK = 8;
 // y_r = sum over p in [ptr[r], ptr[r+1]) of term(p); term(p) is a product
-template <bool STAGED, class F>
+template <class F>
 __device__ __forceinline__ void csr_rows(int64_t m, const int64_t *__restrict__ ptr, double *__restrict__ y, F term) {
-  if constexpr (!STAGED) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    double s = 0.0;
-    for (int64_t k = ptr[i]; k < ptr[i + 1]; k++) s += term(k);
-    y[i] = s;
-    return;
-  }
   __shared__ double prod[CSR_CHUNK];
+  __shared__ unsigned long long longest;
   const int64_t r0 = (int64_t)logical_block(1) * CSR_ROWS;
   if (r0 >= m) return; // the whole block (the grid is rounded up to a multiple of 8)
   const int64_t r1 = r0 + CSR_ROWS < m ? r0 + CSR_ROWS : m;
   const int64_t r = r0 + threadIdx.x;
-  const int64_t q1 = ptr[r1];
+  const int64_t q0 = ptr[r0], q1 = ptr[r1];
   const int64_t p0 = r < r1 ? ptr[r] : q1, p1 = r < r1 ? ptr[r + 1] : q1;
   double s = 0.0;
-  for (int64_t c0 = ptr[r0]; c0 < q1; c0 += CSR_CHUNK) {
+  if (q1 - q0 > CSR_WALK * CSR_CHUNK) {
+    if (threadIdx.x == 0) longest = 0;
+    __syncthreads();
+    atomicMax(&longest, (unsigned long long)(p1 - p0));
+    __syncthreads();
+    if (q1 - q0 > CSR_WALK * (int64_t)longest) {
+      for (int64_t p = p0; p < p1; p++) s += term(p);
+      if (r < r1) y[r] = s;
+      return;
+    }
+  }
+  for (int64_t c0 = q0; c0 < q1; c0 += CSR_CHUNK) {
     const int64_t c1 = c0 + CSR_CHUNK < q1 ? c0 + CSR_CHUNK : q1;
 #pragma unroll
     for (int k = 0; k < CSR_CHUNK / 256; k++) {
@@ -1308,22 +1316,21 @@ __device__ __forceinline__ void csr_rows(int64_t m, const int64_t *__restrict__ 
   if (r < r1) y[r] = s;
 }
 
-template <bool STAGED>
 __global__ __launch_bounds__(256) void k_csr_vmult(int64_t m, const int64_t *__restrict__ rp,
                                                    const int32_t *__restrict__ col,
                                                    const double *__restrict__ val,
                                                    const double *__restrict__ x, double *__restrict__ y) {
-  csr_rows<STAGED>(m, rp, y, [&](int64_t p) { return val[p] * x[col[p]]; });
+  csr_rows(m, rp, y, [&](int64_t p) { return val[p] * x[col[p]]; });
 }
 
 // K: the width of the entry positions, 32 bits when the matrix has fewer
 // than 2^31 entries
-template <bool STAGED, class K>
+template <class K>
 __global__ __launch_bounds__(256) void k_csr_tvmult(int64_t n, const int64_t *__restrict__ tptr,
                                                     const int32_t *__restrict__ trow, const K *__restrict__ tk,
                                                     const double *__restrict__ val,
                                                     const double *__restrict__ x, double *__restrict__ y) {
-  csr_rows<STAGED>(n, tptr, y, [&](int64_t p) { return val[tk[p]] * x[trow[p]]; });
+  csr_rows(n, tptr, y, [&](int64_t p) { return val[tk[p]] * x[trow[p]]; });
 }
 #pragma clang fp contract(on)
 
@@ -1354,11 +1361,8 @@ extern "C" int afe_matrix_tvmult(afe_matrix *a, const double *d_x, double *d_y) 
   auto go = [&](auto kern, const auto *tk) {
     kern<<<csr_grid(a->n), 256, 0, a->ctx->stream>>>(a->n, a->t_ptr.p, a->t_row.p, tk, a->val.p, d_x, d_y);
   };
-  const bool staged = a->nnz <= CSR_LONG_ROWS * a->n;
-  if (a->t_k.p)
-    staged ? go(k_csr_tvmult<true, int64_t>, a->t_k.p) : go(k_csr_tvmult<false, int64_t>, a->t_k.p);
-  else
-    staged ? go(k_csr_tvmult<true, int32_t>, a->t_k32.p) : go(k_csr_tvmult<false, int32_t>, a->t_k32.p);
+  if (a->t_k.p) go(k_csr_tvmult<int64_t>, a->t_k.p);
+  else go(k_csr_tvmult<int32_t>, a->t_k32.p);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(a->ctx->stream));
   API_END
@@ -1369,10 +1373,7 @@ extern "C" int afe_matrix_vmult(afe_matrix *a, const double *d_x, double *d_y) {
   if (!a || !d_x || !d_y) return fail(AFE_E_ARG, "null argument");
   std::lock_guard<CtxMutex> lk(a->ctx->mu);
   HIPCHK(hipSetDevice(a->ctx->device));
-  auto go = [&](auto kern) {
-    kern<<<csr_grid(a->m), 256, 0, a->ctx->stream>>>(a->m, a->rp(), a->col(), a->val.p, d_x, d_y);
-  };
-  a->nnz <= CSR_LONG_ROWS * a->m ? go(k_csr_vmult<true>) : go(k_csr_vmult<false>);
+  k_csr_vmult<<<csr_grid(a->m), 256, 0, a->ctx->stream>>>(a->m, a->rp(), a->col(), a->val.p, d_x, d_y);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(a->ctx->stream));
   API_END

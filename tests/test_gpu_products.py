@@ -1,8 +1,9 @@
 """GPU: A x and A^T x of CSR matrices against the sequential sums, bit for bit
 (products rounded, then added in stored order; the transposed product in
 ascending row order): rows around the staged form's block of 256 rows and chunk
-of 2048 products, rows far longer than the others, and rows long enough on
-average for the one-thread form."""
+of 2048 products, rows far longer than the others, and blocks of rows long
+enough for the one-thread form: beyond 8 chunks of entries, and beyond 8 times
+the longest row, with rows shorter and longer than a chunk."""
 import numpy as np
 import pytest
 
@@ -18,7 +19,9 @@ def _matrix(m, lens, rng):
 
 
 @pytest.mark.parametrize("m,lens", [(1, 1), (255, 3), (256, 8), (257, 8), (600, 64), (520, 65), (300, 300),
-                                    (700, "one long"), (1000, "mixed")])
+                                    (700, "one long"), (1000, "mixed"), (3000, "1 of 3000"), (3000, "5 of 3000"),
+                                    (3000, "7 of 3000"), (3000, "8 of 3000"), (3000, "60 of 3000"),
+                                    (3000, "30 of 500"), (3000, "40 of 500")])
 def test_products_are_the_sequential_sums(ctx, monkeypatch, m, lens):
     import afepack_amd as afe
     print(f"case products m={m} lens={lens}", flush=True)
@@ -26,7 +29,12 @@ def test_products_are_the_sequential_sums(ctx, monkeypatch, m, lens):
     if lens == "one long":
         lens = np.full(m, 5)
         lens[m // 2] = m
-    elif lens == "mixed":
+    elif lens != "mixed" and isinstance(lens, str):  # that many long rows together, across a block's end
+        k, n = (int(v) for v in lens.split(" of "))
+        lens = np.full(m, 5)
+        lens[500:500 + k] = n
+        lens[1100:1100 + k] = n
+    elif isinstance(lens, str):
         lens = rng.integers(1, 60, m)
     rp, col, val = _matrix(m, lens, rng)
     A = afe.Matrix(ctx=ctx, csr=(rp, col, val))
