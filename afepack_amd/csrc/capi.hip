@@ -111,10 +111,11 @@ struct afe_ctx {
   int64_t lds_bytes = 0;    // LDS granted to the coarse-tail workgroup
   std::map<void *, int64_t> user_bytes; // afe_dev_alloc buffers
   int64_t most_bytes = 0; // bound on `bytes` for the library's own buffers (0: none)
-  // device workspace of one call (call_scratch), kept between calls; used
+  // device workspace of one call (CallScratch), kept between calls; used
   // with the context lock held and idle when the lock is released
   double *scratch = nullptr;
   size_t scratch_n = 0;
+  bool scratch_busy = false;
   bool keep_scratch = true;
   double *h_red = nullptr; // pinned: the result of a reduction, written by its kernel
 };
@@ -125,6 +126,19 @@ static bool has_room(const afe_ctx *c, int64_t more) { return c->most_bytes == 0
 // device bytes allocated minus freed by the calling thread (the server
 // measures what one request's set-up keeps)
 static thread_local int64_t t_dev_bytes = 0;
+// gives the kept workspace back unless a call uses it (an allocation that
+// found no room then tries again); false when there was none to give
+static bool give_back_scratch(afe_ctx *c) {
+  std::unique_lock<CtxMutex> lk(c->mu, std::try_to_lock);
+  if (!lk.owns_lock() || !c->scratch || c->scratch_busy) return false;
+  (void)hipFree(c->scratch);
+  c->bytes -= (int64_t)(c->scratch_n * sizeof(double));
+  t_dev_bytes -= (int64_t)(c->scratch_n * sizeof(double));
+  c->scratch = nullptr;
+  c->scratch_n = 0;
+  return true;
+}
+
 // hierarchies built by the calling thread colour every level first-fit in
 // index order (DSatur's fewer colours cost host time a busy set-up pool
 // cannot spare; the server's set-up threads set it)
@@ -183,9 +197,16 @@ template <class T> struct DevBuf {
     release();
     ctx = c;
     if (count == 0) return;
-    const hipError_t e = !has_room(c, count * sizeof(T)) ? hipErrorOutOfMemory
-                         : stream_ordered_alloc()        ? hipMallocAsync((void **)&p, count * sizeof(T), c->stream)
-                                                         : hipMalloc((void **)&p, count * sizeof(T));
+    auto get = [&] {
+      return !has_room(c, count * sizeof(T)) ? hipErrorOutOfMemory
+             : stream_ordered_alloc()        ? hipMallocAsync((void **)&p, count * sizeof(T), c->stream)
+                                             : hipMalloc((void **)&p, count * sizeof(T));
+    };
+    hipError_t e = get();
+    if (e != hipSuccess && give_back_scratch(c)) {
+      (void)hipGetLastError();
+      e = get();
+    }
     if (e != hipSuccess) {
       p = nullptr;
       (void)hipGetLastError();
@@ -205,33 +226,41 @@ template <class T> struct DevBuf {
 // The workspace of a call that returns with the stream synchronised (element
 // loads, partial sums): n doubles from the context's kept buffer, which grows
 // to the largest call's need up to CALL_SCRATCH_MAX, lives as long as the
-// context and counts in its device bytes.  A larger need, or a context that
+// context, or until another allocation finds no room without it, and counts in
+// the context's device bytes.  A larger need, or a context that
 // keeps none (the server's, whose budget counts every byte), takes a buffer of
 // its own for the call.  Allocating and freeing 100 MB took 0.2 ms of the load
 // of a 4.2M-DOF P2 system.
 constexpr size_t CALL_SCRATCH_MAX = (size_t)64 << 20; // doubles (512 MiB)
-static double *call_scratch(afe_ctx *c, size_t n, DevBuf<double> &own) {
-  if (!c->keep_scratch || n > CALL_SCRATCH_MAX) {
-    own.alloc(c, n);
-    return own.p;
-  }
-  if (c->scratch_n < n) {
-    if (c->scratch) {
-      HIPCHK(hipFree(c->scratch));
-      c->bytes -= (int64_t)(c->scratch_n * sizeof(double));
-      c->scratch = nullptr;
-      c->scratch_n = 0;
+class CallScratch {
+  afe_ctx *ctx;
+  DevBuf<double> own;
+
+public:
+  double *p;
+  CallScratch(afe_ctx *c, size_t n) : ctx(c) {
+    if (!c->keep_scratch || c->scratch_busy || n > CALL_SCRATCH_MAX) {
+      own.alloc(c, n);
+      p = own.p;
+      return;
     }
-    if (!has_room(c, n * sizeof(double)) || hipMalloc((void **)&c->scratch, n * sizeof(double)) != hipSuccess) {
-      c->scratch = nullptr;
-      (void)hipGetLastError();
-      throw afe::Error{AFE_E_NOMEM, "device allocation of " + std::to_string(n * sizeof(double)) + " bytes failed"};
+    if (c->scratch_n < n) {
+      (void)give_back_scratch(c);
+      own.alloc(c, n);
+      c->scratch = own.p; // the context's from here on, its bytes are counted
+      c->scratch_n = n;
+      own.p = nullptr;
+      own.n = 0;
     }
-    c->scratch_n = n;
-    c->bytes += (int64_t)(n * sizeof(double));
+    c->scratch_busy = true;
+    p = c->scratch;
   }
-  return c->scratch;
-}
+  CallScratch(const CallScratch &) = delete;
+  CallScratch &operator=(const CallScratch &) = delete;
+  ~CallScratch() {
+    if (!own.p) ctx->scratch_busy = false;
+  }
+};
 
 static inline unsigned nblk(int64_t n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
@@ -427,7 +456,12 @@ extern "C" int afe_dev_alloc(afe_ctx *c, int64_t bytes, void **d_ptr) {
   HIPCHK(hipSetDevice(c->device));
   *d_ptr = nullptr;
   if (bytes == 0) return AFE_OK;
-  if (hipMalloc(d_ptr, (size_t)bytes) != hipSuccess) {
+  hipError_t e = hipMalloc(d_ptr, (size_t)bytes);
+  if (e != hipSuccess && give_back_scratch(c)) {
+    (void)hipGetLastError();
+    e = hipMalloc(d_ptr, (size_t)bytes);
+  }
+  if (e != hipSuccess) {
     (void)hipGetLastError();
     *d_ptr = nullptr;
     return fail(AFE_E_NOMEM, "hipMalloc failed");
@@ -1428,9 +1462,10 @@ extern "C" int afe_rhs(afe_space *s, int32_t acc, int32_t fkind, const afe_field
   if (!q) return fail(AFE_E_ARG, "no quadrature rule of that accuracy");
   std::lock_guard<CtxMutex> lk(s->ctx->mu);
   HIPCHK(hipSetDevice(s->ctx->device));
-  DevBuf<double> fstore, own;
+  DevBuf<double> fstore;
   FieldDev fd = upload_field(s->ctx, fkind == AFE_F_VARCOEF ? coef : nullptr, fstore);
-  double *Fe = call_scratch(s->ctx, (size_t)s->h.n_elem * s->h.n_loc, own);
+  CallScratch scratch(s->ctx, (size_t)s->h.n_elem * s->h.n_loc);
+  double *Fe = scratch.p;
   switch (s->h.kind) {
   case P1_TRI: launch_loads<P1_TRI>(s, q, fkind, fd, d_nodal, Fe); break;
   case P2_TRI: launch_loads<P2_TRI>(s, q, fkind, fd, d_nodal, Fe); break;
@@ -1495,9 +1530,10 @@ extern "C" int afe_rhs_qp(afe_space *s, int32_t acc, const double *h_fq, double 
   std::lock_guard<CtxMutex> lk(s->ctx->mu);
   HIPCHK(hipSetDevice(s->ctx->device));
   const int64_t ne = s->h.n_elem;
-  DevBuf<double> fq, own;
+  DevBuf<double> fq;
   fq.upload(s->ctx, h_fq, (size_t)ne * q->n);
-  double *Fe = call_scratch(s->ctx, (size_t)ne * s->h.n_loc, own);
+  CallScratch scratch(s->ctx, (size_t)ne * s->h.n_loc);
+  double *Fe = scratch.p;
   const double *qd = s->ctx->d_quad + q->off;
   hipStream_t st = s->ctx->stream;
   switch (s->h.kind) {
@@ -1626,8 +1662,8 @@ static int fe_error(afe_space *s, const double *d_uh, int acc, int h1, double *e
   if (!q) return fail(AFE_E_ARG, "no quadrature rule of that accuracy");
   std::lock_guard<CtxMutex> lk(s->ctx->mu);
   HIPCHK(hipSetDevice(s->ctx->device));
-  DevBuf<double> own;
-  double *part = call_scratch(s->ctx, RED_BLOCKS, own);
+  CallScratch scratch(s->ctx, RED_BLOCKS);
+  double *part = scratch.p;
   const unsigned nb = std::min<unsigned>(nblk(s->h.n_elem), RED_BLOCKS);
   switch (s->h.kind) {
   case P1_TRI: launch_error<P1_TRI>(s, q, h1, d_uh, nb, part); break;
@@ -2146,11 +2182,11 @@ static void build_dense(afe_amg *g, int ld, int lc, const double *minv, int coar
   const int cols = std::min(n, DENSE_COLUMNS);
   DevBuf<LevelDev<double>> tl;
   DevBuf<TailJob<double>> jobs;
-  DevBuf<double> own;
   out.alloc(ctx, (size_t)n * n);
   tl.alloc(ctx, (size_t)cols * nl);
   jobs.alloc(ctx, cols);
-  double *W = call_scratch(ctx, (size_t)cols * stride, own);
+  CallScratch scratch(ctx, (size_t)cols * stride);
+  double *W = scratch.p;
   const int lds_cap = (int)ctx->lds_bytes;
   for (int c0 = 0; c0 < n; c0 += cols) {
     const int m = std::min(cols, n - c0);
@@ -2297,8 +2333,8 @@ static void form_sweeps(afe_amg *g) {
     words += w.head.size() + w.counts.size() + (size_t)2 * w.nb * 2 * w.W;
   }
   if (work.empty()) return;
-  DevBuf<double> own;
-  int32_t *at = reinterpret_cast<int32_t *>(call_scratch(ctx, (words + 1) / 2, own));
+  CallScratch scratch(ctx, (words + 1) / 2);
+  int32_t *at = reinterpret_cast<int32_t *>(scratch.p);
   for (Work &w : work) {
     w.d_head = at;
     at += w.head.size();

@@ -3,7 +3,9 @@ the small levels' sub-cycle, the tables of the block sweeps): the cycle is the
 one of a hierarchy that has these turned off, bit for bit, nothing of them stays
 allocated, and after a refresh with room the cycle is the one of a hierarchy
 that never ran short.  The shortage is AFE_DEVICE_BYTES, which bounds a
-context's own buffers; the vector `ballast` makes the room afterwards."""
+context's own buffers; the vector `ballast` makes the room afterwards.
+
+And a context's kept workspace, which makes room for other allocations."""
 import numpy as np
 import pytest
 
@@ -71,3 +73,42 @@ def test_first_cycle_without_room(monkeypatch, dense, sweeps, some):
     free.g.lazy_reinit(free.A)
     for a, b in zip(run.cycles(), free.cycles()):
         assert np.array_equal(a, b)
+
+
+def test_kept_workspace_makes_room(monkeypatch):
+    """A load keeps its element loads' buffer; the matrix assembled next finds
+    room only without it, and a later load has none then."""
+    import afepack_amd as afe
+    print("case memory workspace", flush=True)
+    c, ev, vm = make_mesh(1, 60, 0.05, 3)
+
+    def parts(ctx):
+        held = [ctx.device_bytes()]
+        sp = afe.Space(ctx, 1, c, ev, vm)
+        b = afe.DeviceVector(ctx, sp.n_dof)
+        held.append(ctx.device_bytes())
+        sp.rhs(2, afe.F_POISSON, out=b)
+        held.append(ctx.device_bytes())
+        A = afe.Matrix(sp)
+        A.assemble(afe.OP_STIFF, 2)
+        held.append(ctx.device_bytes())
+        first = b.numpy()
+        sp.rhs(2, afe.F_POISSON, out=b)
+        assert np.array_equal(b.numpy(), first)
+        return held, A.values()
+
+    monkeypatch.delenv("AFE_DEVICE_BYTES", raising=False)
+    (_, h1, h2, h3), want = parts(afe.Context(0))
+    work = h2 - h1
+    assert work >= 8 * 3 * 7200
+    monkeypatch.setenv("AFE_DEVICE_BYTES", str(h3 - 1))
+    ctx = afe.Context(0)
+    with pytest.raises(afe.AfeError):  # the load that follows has no room
+        parts(ctx)
+    ctx = afe.Context(0)
+    sp = afe.Space(ctx, 1, c, ev, vm)
+    b = sp.rhs(2, afe.F_POISSON)
+    A = afe.Matrix(sp)
+    A.assemble(afe.OP_STIFF, 2)
+    assert np.array_equal(A.values(), want)
+    assert ctx.device_bytes() == h3 - work
