@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <numeric>
 #include <queue>
 #include <tuple>
@@ -399,7 +400,8 @@ void transpose_map(int64_t m, int64_t n, const std::vector<int64_t> &rp, const s
   for (int64_t j = 0; j < n; j++) tptr[j + 1] += tptr[j];
   trow.resize(nnz);
   tk.resize(nnz);
-  std::vector<int64_t> fill(tptr.begin(), tptr.end() - 1); // here: no allocation may fail in a thread
+  // (here: no allocation may fail in a thread; each fills its own range)
+  const std::unique_ptr<int64_t[]> fill(new int64_t[n]);
 #pragma omp parallel
   {
     const int64_t T = omp_get_num_threads(), t = omp_get_thread_num();
@@ -407,6 +409,7 @@ void transpose_map(int64_t m, int64_t n, const std::vector<int64_t> &rp, const s
       return s == T ? n : std::lower_bound(tptr.begin(), tptr.end(), nnz * s / T) - tptr.begin();
     };
     const int64_t j0 = bound(t), j1 = bound(t + 1);
+    for (int64_t j = j0; j < j1; j++) fill[j] = tptr[j];
     for (int64_t i = 0; i < m && j0 < j1; i++)
       for (int64_t k = rp[i]; k < rp[i + 1]; k++) {
         const int64_t j = col[k];
