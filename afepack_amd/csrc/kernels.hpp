@@ -108,8 +108,10 @@ template <int D, bool GRAD> __device__ __forceinline__ double field_g(const Fiel
 
 // The element kernels below follow the reference's arithmetic step by step
 // (the plugins of element_geom.hpp, Jxw = w * jacobian * volume, K(j,k) +=
-// Jxw * <g_j, g_k>) with floating-point contraction off, so each element
-// matrix is bit-identical to the host restatement.
+// Jxw * <g_j, g_k>) with floating-point contraction off, so the stiffness and
+// mass matrices of each element are bit-identical to the host restatement.  The
+// variable coefficient agrees with it to rounding: its sines are this file's,
+// and the P1 forms sum it over the points before the inner products.
 #pragma clang fp contract(off)
 
 // ---------------------------------------------------------------------------
@@ -711,7 +713,7 @@ __global__ __launch_bounds__(256) void k_gather_vec(int64_t n, int xcd, const in
 // are depends on the pattern and the marks only: the space lists the marked
 // rows and the positions of their off-diagonals and of the entries in their
 // columns once, and the elimination touches nothing else.  4.2M P2 DOFs, 8192
-// of them marked: 152 -> 5.5 us (a pass over every row's columns and their
+// of them marked: 150 -> 5.7 us (a pass over every row's columns and their
 // marks before).
 __global__ __launch_bounds__(256) void k_dirichlet_zero(int64_t n_rows, const int32_t *__restrict__ rows,
                                                         const int64_t *__restrict__ rp, int64_t n_pos,
