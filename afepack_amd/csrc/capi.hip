@@ -2333,8 +2333,16 @@ static void form_sweeps(afe_amg *g) {
     words += w.head.size() + w.counts.size() + (size_t)2 * w.nb * 2 * w.W;
   }
   if (work.empty()) return;
-  CallScratch scratch(ctx, (words + 1) / 2);
-  int32_t *at = reinterpret_cast<int32_t *>(scratch.p);
+  // a buffer of its own, once a hierarchy: 27 MB for 131K rows
+  DevBuf<int32_t> buf;
+  buf.alloc(ctx, words);
+  // also where an allocation below fails: the copies end before their host
+  // vectors and this buffer go
+  struct Wait {
+    hipStream_t st;
+    ~Wait() { (void)hipStreamSynchronize(st); }
+  } wait{st};
+  int32_t *at = buf.p;
   for (Work &w : work) {
     w.d_head = at;
     at += w.head.size();
@@ -2436,7 +2444,7 @@ static void form_sweeps(afe_amg *g) {
         d.sweep_col_slice.p, d.sweep_cols.p, d.sweep_src.p);
   }
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(st)); // the workspace is free again
+  HIPCHK(hipStreamSynchronize(st));
 }
 
 template <class T> static DevBuf<T> &sweep_buf(DevLevel &d);
@@ -3338,14 +3346,14 @@ extern "C" int afe_amg_solve(afe_amg *g, double *d_x, const double *d_r, double 
   if (rtol <= 0 && !(mode & 2) && !verbose()) {
     // the reference's form (no early exit, nothing printed per cycle): the
     // step + 1 cycles run back to back, the residual is taken once after them
-    for (; it <= step; it++) launch_graph_or_issue(g, 0, false, g->prm.smooth, step + 1 - it);
+    for (; it <= step; it++) launch_graph_or_issue(g, 0, false, g->prm.smooth, std::min<int64_t>(step - it, DENSE_CYCLES) + 1);
     residual_norms(g, false, d0.b64.p, d0.x64.p, nullptr);
     read_scalars(g);
     rr = g->h_sc->rr;
     l1 = g->h_sc->l1;
   } else {
     while (true) {
-      launch_graph_or_issue(g, 0, false, g->prm.smooth, step + 1 - it);
+      launch_graph_or_issue(g, 0, false, g->prm.smooth, std::min<int64_t>(step - it, DENSE_CYCLES) + 1);
       residual_norms(g, false, d0.b64.p, d0.x64.p, nullptr);
       read_scalars(g);
       rr = g->h_sc->rr;
@@ -3397,7 +3405,7 @@ constexpr int CG_SUM_PARTIALS = 4096;
 
 // z = M^{-1} r with one symmetric V-cycle from zero; r and z in the natural
 // numbering, the V-cycle in the level-0 colour order
-template <class T> static void precondition_perm(afe_amg *g, const double *r, bool first, int ahead) {
+template <class T> static void precondition_perm(afe_amg *g, const double *r, bool first, int64_t ahead) {
   DevLevel &d0 = g->lv[0];
   hipStream_t s = g->ctx->stream;
   const int64_t n = d0.n;
@@ -3562,7 +3570,7 @@ static int pcg_impl(afe_amg *g, double *d_x, const double *d_b, double rtol, int
   for (int outer = 0; outer < 4; outer++) {
   while (!conv && it < max_it) {
     k_fill<double><<<nblk(n), 256, 0, s>>>(n, g->wp.p, 0.0);
-    precondition_perm<T>(g, g->wr.p, true, max_it - it + 1);
+    precondition_perm<T>(g, g->wr.p, true, (int64_t)max_it - it + 1);
     while (it < max_it) {
       launch_cg_iteration<T>(g);
       HIPCHK(hipEventSynchronize(g->it_ev));

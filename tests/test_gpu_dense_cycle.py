@@ -131,6 +131,10 @@ def test_which_cycles_form_the_matrix(ctx):
     x.zero()
     g.pcg(x, b, rtol=1e-8, max_it=100, prec=afe.PREC_FP32)
     assert formed() == (False, True)
+    g.lazy_reinit(A)
+    x.zero()
+    g.pcg(x, b, rtol=1e-8, max_it=2**31 - 1, prec=afe.PREC_FP32)  # the largest bound
+    assert formed() == (False, True)
     # the step form and the matrix agree along one call's cycles (captured both ways)
     ref = afe.DeviceVector(ctx, sp.n_dof)
     g.vcycle(ref, b, afe.PREC_FP64)
