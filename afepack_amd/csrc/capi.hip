@@ -2295,8 +2295,9 @@ static void drop_sweep(DevLevel &d) {
 // so that hierarchies which only join a batch never pay for it.
 // Creating a hierarchy takes what it takes without tables, 94 ms on 263K P2
 // DOFs, 125 on 251K P1 and 41 on 58K P2 (113, 145 and 56 with tables built on
-// the host for each); the first solve takes 2.3, 3.6 and 2.6 ms longer than
-// the second, about half of it the partition.
+// the host for each); the first solve takes 3.0, 3.9 and 3.0 ms longer than
+// the second (with graphs and the dense sub-cycle, 0.9, 0.8 and 0.8 of it),
+// about half of it the partition.
 static void form_sweeps(afe_amg *g) {
   afe_ctx *ctx = g->ctx;
   hipStream_t st = ctx->stream;
