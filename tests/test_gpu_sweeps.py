@@ -142,3 +142,33 @@ def test_levels_with_large_closures_keep_the_colour_launches(ctx, monkeypatch):
         assert g.sweep_info()[0]["blocks"] == 0
         out.append(z.numpy())
     assert np.array_equal(out[0], out[1])
+
+
+def test_blocks_that_fit_in_lds_in_fp32_only(ctx, monkeypatch):
+    """85184 rows of tetrahedra: a block's arrays take 98 KB in FP32 and 168 KB,
+    more than a workgroup has, in FP64.  FP64 cycles keep the colour launches,
+    bit for bit; FP32 ones take the blocks."""
+    import afepack_amd as afe
+    print("case sweeps fp32 only", flush=True)
+    c, ev, vm = make_mesh(3, 43, 0.05, 21)
+    sp = afe.Space(ctx, 3, c, ev, vm)
+    A = afe.Matrix(sp)
+    A.assemble(afe.OP_STIFF, 2)
+    b = sp.rhs(2, afe.F_POISSON)
+    A.apply_dirichlet(b)
+    prm = afe.AmgParams(lazy=1, smooth=1, build_fp32=1)
+    rng = np.random.default_rng(2)
+    r = afe.DeviceVector.from_numpy(ctx, rng.uniform(-1, 1, sp.n_dof))
+    out = []
+    for rows in ("0", "131072"):
+        monkeypatch.setenv("AFE_SWEEP_ROWS", rows)
+        g = afe.Amg(A, prm)
+        z = afe.DeviceVector(ctx, sp.n_dof)
+        for prec in (afe.PREC_FP32, afe.PREC_FP64):
+            g.vcycle(z, r, prec)
+            out.append(z.numpy())
+        v = g.sweep_info()[0]
+        assert (v["blocks"] > 1, v["fused"]) == (rows != "0", (False, rows != "0"))
+    assert np.array_equal(out[1], out[3])
+    assert not np.array_equal(out[0], out[2])
+    assert np.linalg.norm(out[0] - out[2]) <= 1e-5 * np.linalg.norm(out[0])
